@@ -188,14 +188,12 @@ private:
     std::vector<std::string> order_;
 };
 
-// Concatenated node-linear tiles of every receiver tile of the graph.
+// Concatenated node-linear rows and sets of every receiver tile of the graph.
 struct PlanSet {
-    std::vector<GemmTile> tiles;
-    std::vector<std::size_t> tile_begin;  // per receiver tile: first GemmTile
-    std::vector<int> rows;                // packed (local node << 4 | m)
-    std::vector<GemmTileSet> sets;        // per receiver tile, tiles relative to its first
-    std::vector<std::size_t> set_begin;
-    DevBuf d_tiles, d_rows, d_sets;
+    std::vector<int> rows;          // packed (local node << 4 | m)
+    std::vector<GemmTileSet> sets;
+    std::vector<std::size_t> set_begin;  // per receiver tile: its first set
+    DevBuf d_rows, d_sets;
 };
 
 }  // namespace
@@ -444,21 +442,21 @@ struct Evaluator {
         dm.R1c = reinterpret_cast<const float4*>(put(hm.R1_coef));
         dm.H0 = put(hm.H0);
         const std::size_t a0_blocks = static_cast<std::size_t>(hm.num_elements) * (hm.l_max + 1);
-        dm.A0_w = put(swizzled(hm.A0_w, a0_blocks, hm.C, hm.C));
-        dm.A0_wt = put(swizzled(hm.A0_wt, a0_blocks, hm.C, hm.C));
+        dm.A0_w = put_gemm(hm.A0_w, a0_blocks, hm.C, hm.C);
+        dm.A0_wt = put_gemm(hm.A0_wt, a0_blocks, hm.C, hm.C);
         dm.m0_terms = put(hm.m0_terms);
         dm.m0_toff = put(hm.m0_term_offset);
         dm.m0_term_offset = hm.m0_term_offset;
         dm.T0 = static_cast<int>(hm.m0_terms.size());
         dm.m0_coef = put(hm.m0_coef);
-        dm.H1_w = put(swizzled(hm.H1_w, hm.L_max + 1, hm.C, hm.C));
-        dm.H1_wt = put(swizzled(hm.H1_wt, hm.L_max + 1, hm.C, hm.C));
+        dm.H1_w = put_gemm(hm.H1_w, hm.L_max + 1, hm.C, hm.C);
+        dm.H1_wt = put_gemm(hm.H1_wt, hm.L_max + 1, hm.C, hm.C);
         dm.pre_linear_up = hm.pre_linear_up;
         dm.residual = hm.residual;
         dm.single_layer = hm.single_layer;
         if (hm.pre_linear_up) {
-            dm.P0_w = put(swizzled(hm.P0, 1, hm.C, hm.C));
-            dm.P0_wt = put(swizzled(hm.P0t, 1, hm.C, hm.C));
+            dm.P0_w = put_gemm(hm.P0, 1, hm.C, hm.C);
+            dm.P0_wt = put_gemm(hm.P0t, 1, hm.C, hm.C);
         }
         if (hm.residual) {
             dm.res_H1 = put(hm.res_H1);
@@ -467,12 +465,12 @@ struct Evaluator {
         dm.field = hm.field;
         if (hm.field) {
             const int nl = hm.L_max + 1, np = static_cast<int>(hm.field_paths.size());
-            dm.P_w = put(swizzled(hm.P_all, nl, hm.C, hm.C));
-            dm.P_wt = put(swizzled(hm.P_allt, nl, hm.C, hm.C));
-            dm.U_w = put(swizzled(hm.U_all, nl, hm.C, hm.C));
-            dm.U_wt = put(swizzled(hm.U_allt, nl, hm.C, hm.C));
-            dm.field_W = put(swizzled(hm.field_W, np, hm.C, hm.C));
-            dm.field_Wt = put(swizzled(hm.field_Wt, np, hm.C, hm.C));
+            dm.P_w = put_gemm(hm.P_all, nl, hm.C, hm.C);
+            dm.P_wt = put_gemm(hm.P_allt, nl, hm.C, hm.C);
+            dm.U_w = put_gemm(hm.U_all, nl, hm.C, hm.C);
+            dm.U_wt = put_gemm(hm.U_allt, nl, hm.C, hm.C);
+            dm.field_W = put_gemm(hm.field_W, np, hm.C, hm.C);
+            dm.field_Wt = put_gemm(hm.field_Wt, np, hm.C, hm.C);
             if (hm.residual) dm.res_pre = put(hm.res_pre);
             // Z rows: each path's l_in m's in turn; Y rows: its l_out m's
             std::vector<int> zoff(np + 1, 0), yoff(np + 1, 0);
@@ -493,15 +491,15 @@ struct Evaluator {
         }
         dm.cg = put(hm.cg_dense);
         {
-            std::vector<float> w(hm.A1_w.size()), wt(hm.A1_wt.size());
+            std::vector<GemmBlocks> f, r;
             for (int l = 0; l <= hm.l_max; ++l) {
                 const int K = hm.num_e[l] * hm.C;
                 if (K == 0) continue;
-                swizzle_gemm_weights(hm.A1_w.data() + hm.A1_offset[l], K, hm.C, w.data() + hm.A1_offset[l]);
-                swizzle_gemm_weights(hm.A1_wt.data() + hm.A1_offset[l], hm.C, K, wt.data() + hm.A1_offset[l]);
+                f.push_back({hm.A1_offset[l], 1, K, hm.C});
+                r.push_back({hm.A1_offset[l], 1, hm.C, K});
             }
-            dm.A1_w = put(w);
-            dm.A1_wt = put(wt);
+            dm.A1_w = put_gemm(hm.A1_w, f);
+            dm.A1_wt = put_gemm(hm.A1_wt, r);
         }
         dm.A1_offset = hm.A1_offset;
         dm.num_e = hm.num_e;
@@ -521,12 +519,30 @@ struct Evaluator {
         dm.E0 = put(hm.atomic_energies);
     }
 
-    // blocks [count][K][N] of a weight array in the MFMA operand order
-    static std::vector<float> swizzled(const std::vector<float>& w, std::size_t count, int K, int N) {
-        std::vector<float> out(w.size());
-        const std::size_t blk = static_cast<std::size_t>(K) * N;
-        for (std::size_t b = 0; b < count; ++b) swizzle_gemm_weights(w.data() + b * blk, K, N, out.data() + b * blk);
-        return out;
+    // count blocks [K][N] of a weight array from element offset `first`
+    struct GemmBlocks {
+        std::int64_t first;
+        std::size_t count;
+        int K, N;
+    };
+    // a weight array on the device in the GEMM kernels' operand orders
+    GemmWeights put_gemm(const std::vector<float>& w, const std::vector<GemmBlocks>& blocks) {
+        DevBuf raw;
+        const float* src = upload(raw, w, stream);
+        model_bufs.push_back(std::make_unique<DevBuf>());
+        char* dst = static_cast<char*>(model_bufs.back()->ensure(std::max<std::size_t>(1, w.size()) * 6));
+        std::vector<float> waves(w.size());
+        for (const auto& b : blocks) {
+            launch_pack_gemm_weights(src + b.first, b.count, b.K, b.N, dst + 6 * b.first, stream);
+            const std::size_t blk = static_cast<std::size_t>(b.K) * b.N;
+            for (std::size_t q = 0; q < b.count; ++q)
+                swizzle_gemm_weights(w.data() + b.first + q * blk, b.K, b.N, waves.data() + b.first + q * blk);
+        }
+        SMX_HIP(hipStreamSynchronize(stream));
+        return GemmWeights{dst, put(waves)};
+    }
+    GemmWeights put_gemm(const std::vector<float>& w, std::size_t count, int K, int N) {
+        return put_gemm(w, {GemmBlocks{0, count, K, N}});
     }
 
     // Weight groups of the node linears: A0 per (type, l), H1 per l, A1 per
@@ -564,7 +580,7 @@ struct Evaluator {
         max_n_a1r = mx(groups_a1r);
         sub_a0 = sub(groups_a0);
         sub_h1 = sub(groups_h1);
-        sub_a1f = sub(groups_a1f);  // (the A1 forward plan prefers 64 columns: K runs to 3C)
+        sub_a1f = sub(groups_a1f);
         sub_a1r = sub(groups_a1r);
         upload(d_groups_a0, groups_a0, stream);
         upload(d_groups_h1, groups_h1, stream);
@@ -782,10 +798,8 @@ struct Evaluator {
     // one tile over all F feature nodes: the h1 (U, U^T), fz and fy plans
     void build_feature_tile() {
         for (PlanSet* p : {&ps_feat_h1, &ps_feat_fz, &ps_feat_fy}) {
-            p->tiles.clear();
             p->rows.clear();
             p->sets.clear();
-            p->tile_begin.assign(1, 0);
             p->set_begin.assign(1, 0);
         }
         auto add = [&](PlanSet& P, int group, int l) {
@@ -793,12 +807,8 @@ struct Evaluator {
             for (int m = 0; m < 2 * l + 1; ++m)
                 for (int q = 0; q < F; ++q) P.rows.push_back(q << 4 | m);
             const int end = static_cast<int>(P.rows.size());
-            const int t0 = static_cast<int>(P.tiles.size());
-            for (int s0 = start; s0 < end; s0 += kGemmRows)
-                P.tiles.push_back(GemmTile{s0, std::min(kGemmRows, end - s0), group});
-            const int t1 = static_cast<int>(P.tiles.size());
-            for (int t = t0; t < t1; t += kGemmShareWaves)
-                P.sets.push_back(GemmTileSet{t, std::min(kGemmShareWaves, t1 - t)});
+            for (int s0 = start; s0 < end; s0 += kGemmSetRows)
+                P.sets.push_back(GemmTileSet{s0, std::min(kGemmSetRows, end - s0), group});
         };
         for (int l = 0; l <= hm.L_max; ++l) add(ps_feat_h1, l, l);
         for (std::size_t p = 0; p < hm.field_paths.size(); ++p) {
@@ -806,15 +816,11 @@ struct Evaluator {
             add(ps_feat_fy, static_cast<int>(p), hm.field_paths[p].l_out);
         }
         auto view = [&](PlanSet& P, const DevBuf& groups, int max_n, int n_sub) {
-            P.tile_begin.push_back(P.tiles.size());
             P.set_begin.push_back(P.sets.size());
-            upload(P.d_tiles, P.tiles, stream);
             upload(P.d_rows, P.rows, stream);
             upload(P.d_sets, P.sets, stream);
             GemmPlan g;
             g.n_sub = n_sub;
-            g.tiles = P.d_tiles.as<GemmTile>();
-            g.num_tiles = static_cast<int>(P.tiles.size());
             g.groups = groups.as<GemmGroup>();
             g.rows = P.d_rows.as<int>();
             g.max_n = max_n;
@@ -838,8 +844,6 @@ struct Evaluator {
         h_batches.clear();
         batch_begin.clear();
         for (PlanSet* p : {&ps_a0, &ps_h1, &ps_a1f, &ps_a1r, &ps_cap, &ps_fz, &ps_fy}) {
-            p->tiles.clear();
-            p->tile_begin.clear();
             p->rows.clear();
             p->sets.clear();
             p->set_begin.clear();
@@ -855,22 +859,17 @@ struct Evaluator {
             });
             h_node_list.insert(h_node_list.end(), order.begin(), order.end());
             for (PlanSet* p : {&ps_a0, &ps_h1, &ps_a1f, &ps_a1r, &ps_cap, &ps_fz, &ps_fy}) {
-                p->tile_begin.push_back(p->tiles.size());
                 p->set_begin.push_back(p->sets.size());
             }
             // rows (node order[a..b), m in [0, 2l+1)) of one group, cut into
-            // wave tiles, and the tiles into sets of up to kGemmShareWaves
+            // workgroups' sets
             auto add = [&](PlanSet& P, int group, int l, int a, int b) {
                 const int start = static_cast<int>(P.rows.size());
                 for (int m = 0; m < 2 * l + 1; ++m)
                     for (int q = a; q < b; ++q) P.rows.push_back(order[q] << 4 | m);
                 const int end = static_cast<int>(P.rows.size());
-                const int t0 = static_cast<int>(P.tiles.size() - P.tile_begin.back());
-                for (int s0 = start; s0 < end; s0 += kGemmRows)
-                    P.tiles.push_back(GemmTile{s0, std::min(kGemmRows, end - s0), group});
-                const int t1 = static_cast<int>(P.tiles.size() - P.tile_begin.back());
-                for (int t = t0; t < t1; t += kGemmShareWaves)
-                    P.sets.push_back(GemmTileSet{t, std::min(kGemmShareWaves, t1 - t)});
+                for (int s0 = start; s0 < end; s0 += kGemmSetRows)
+                    P.sets.push_back(GemmTileSet{s0, std::min(kGemmSetRows, end - s0), group});
             };
             for (int p = 0; p < t.nr;) {
                 int q = p;
@@ -895,9 +894,7 @@ struct Evaluator {
         }
         batch_begin.push_back(h_batches.size());
         for (PlanSet* p : {&ps_a0, &ps_h1, &ps_a1f, &ps_a1r, &ps_cap, &ps_fz, &ps_fy}) {
-            p->tile_begin.push_back(p->tiles.size());
             p->set_begin.push_back(p->sets.size());
-            upload(p->d_tiles, p->tiles, stream);
             upload(p->d_rows, p->rows, stream);
             upload(p->d_sets, p->sets, stream);
         }
@@ -911,8 +908,6 @@ struct Evaluator {
         auto view = [&](const PlanSet& P, std::size_t ti, const DevBuf& groups, int max_n, int n_sub) {
             GemmPlan g;
             g.n_sub = n_sub;
-            g.tiles = P.d_tiles.as<GemmTile>() + P.tile_begin[ti];
-            g.num_tiles = static_cast<int>(P.tile_begin[ti + 1] - P.tile_begin[ti]);
             g.groups = groups.as<GemmGroup>();
             g.rows = P.d_rows.as<int>();
             g.max_n = max_n;
@@ -924,7 +919,6 @@ struct Evaluator {
             tiles[ti].a0 = view(ps_a0, ti, d_groups_a0, max_n_a0, sub_a0);
             tiles[ti].h1 = view(ps_h1, ti, d_groups_h1, max_n_h1, sub_h1);
             tiles[ti].a1f = view(ps_a1f, ti, d_groups_a1f, max_n_a1f, sub_a1f);
-            tiles[ti].a1f.narrow = true;
             tiles[ti].a1r = view(ps_a1r, ti, d_groups_a1r, max_n_a1r, sub_a1r);
             if (hm.pre_linear_up) {
                 tiles[ti].cap = view(ps_cap, ti, d_groups_cap, hm.C, sub_cap);

@@ -19,6 +19,14 @@ struct FieldEntryDev {
     float coef;
 };
 
+// Weight blocks of the node linears in the operand order of the two GEMM
+// kernels: three bf16 parts per weight (6 bytes, launch_pack_gemm_weights) for
+// the workgroup form, FP32 (swizzle_gemm_weights) for the one-wave form.
+struct GemmWeights {
+    const void* packed = nullptr;
+    const float* fp32 = nullptr;
+};
+
 // Model tables resident in HBM (owned by the evaluator).
 struct DeviceModel {
     int C = 0, l_max = 0, L_max = 0, num_lm = 0, num_LM = 0, num_elements = 0;
@@ -29,40 +37,40 @@ struct DeviceModel {
     const float4* R0c = nullptr;  // [interval][(l_max+1)*C]
     const float4* R1c = nullptr;  // [interval][P*C]
     const float* H0 = nullptr;
-    const float* A0_w = nullptr;
-    const float* A0_wt = nullptr;
+    GemmWeights A0_w;
+    GemmWeights A0_wt;
     const std::int32_t* m0_terms = nullptr;
     const int* m0_toff = nullptr;     // [num_LM+1] term offsets per output
     std::vector<int> m0_term_offset;  // host copy
     int T0 = 0;
     const float* m0_coef = nullptr;
-    const float* H1_w = nullptr;
-    const float* H1_wt = nullptr;
+    GemmWeights H1_w;
+    GemmWeights H1_wt;
     // pre_linear_up basis: x = M0[:,0,:] P0 and M0_adj[:,0,:] += P0 d (GEMM
-    // weights P0 and P0^T, swizzled); residual: per-type H1 and x offsets
+    // weights P0 and P0^T, packed); residual: per-type H1 and x offsets
     bool pre_linear_up = false, residual = false;
     // one interaction: M1 of H1, no R1 / A1 (single_layer_readout)
     bool single_layer = false;
     // MACEField: H1p = M0 P (+ b), H1f = H1p + field terms, x = H1f[:,0,:],
-    // H1 = H1f U (GEMM weights swizzled: P, U per l; W per path)
+    // H1 = H1f U (GEMM weights packed: P, U per l; W per path)
     bool field = false;
-    const float* P_w = nullptr;
-    const float* P_wt = nullptr;
-    const float* U_w = nullptr;
-    const float* U_wt = nullptr;
-    const float* field_W = nullptr;
-    const float* field_Wt = nullptr;
+    GemmWeights P_w;
+    GemmWeights P_wt;
+    GemmWeights U_w;
+    GemmWeights U_wt;
+    GemmWeights field_W;
+    GemmWeights field_Wt;
     const float* res_pre = nullptr;  // [type][NH][C]
     const FieldEntryDev* field_entries = nullptr;
     int num_field_entries = 0;
     int field_zr = 0, field_yr = 0;  // rows of Z and Y per node
-    const float* P0_w = nullptr;
-    const float* P0_wt = nullptr;
+    GemmWeights P0_w;
+    GemmWeights P0_wt;
     const float* res_H1 = nullptr;  // [type][NH][C]
     const float* res_x = nullptr;   // [type][C]
     const float* cg = nullptr;
-    const float* A1_w = nullptr;
-    const float* A1_wt = nullptr;
+    GemmWeights A1_w;
+    GemmWeights A1_wt;
     std::vector<std::int64_t> A1_offset;  // host copy
     std::vector<int> num_e, lme_base;     // host copy
     const std::int32_t* m1_terms = nullptr;
@@ -118,37 +126,30 @@ struct DeviceGraph {
 // Node linears: out[row, n] = sum_k in[row, k] W[k, n] over the rows of one
 // weight group.  A row is (tile-local node, m) packed as node << 4 | m; its
 // input starts at node*in_stride + in_base + m*in_mstride (likewise the
-// output).  W is stored in the MFMA operand order of swizzle_gemm_weights.
+// output).  W is packed by launch_pack_gemm_weights.
 struct GemmGroup {
-    std::int64_t w_off;  // element offset of the group's swizzled [K][N] block
+    std::int64_t w_off;  // element offset of the group's [K][N] block
     int K, N;
     int in_stride, in_base, in_mstride;
     int out_stride, out_base, out_mstride;
 };
-// rows per wave tile (a multiple of 16): 16 rows x up to 128 columns per
-// wave.  At the medium shape this reads each input row once per 128 output
-// columns and still gives about five waves per SIMD; it measured faster than
-// 32 x 64 and 64 x 64 tiles.
-constexpr int kGemmRows = 16;
-struct GemmTile {
-    int row_start, count, group;  // rows [row_start, row_start+count), count <= kGemmRows
-};
-// Up to kGemmShareWaves consecutive tiles of one group: the workgroup of the
-// shared-operand GEMM kernel (tile indices relative to GemmPlan::tiles).
-constexpr int kGemmShareWaves = 8;
+// Up to kGemmSetTiles 16-row tiles of one group: a workgroup of the GEMM
+// kernel, rows [row_start, row_start+count) of the plan's row list.
+constexpr int kGemmSetTiles = 8;
+constexpr int kGemmSetRows = 16 * kGemmSetTiles;
+// workgroups from which a launch takes the workgroup form (one per CU), and
+// from which their column blocks widen (two per CU)
+constexpr long long kGemmWaveFill = 256, kGemmFill = 512;
 struct GemmTileSet {
-    int first, count;
+    int row_start, count, group;
 };
 struct GemmPlan {
-    const GemmTile* tiles = nullptr;
     const GemmGroup* groups = nullptr;
     const int* rows = nullptr;        // packed (node << 4 | m)
-    int num_tiles = 0;
     int max_n = 0;
-    int n_sub = 1;  // 16-column tiles per wave (8, 4, 2 or 1): divides every group's N/16
-    const GemmTileSet* sets = nullptr;  // tiles grouped for the shared-operand kernel
+    int n_sub = 2;  // most 16-column tiles per wave (8, 4 or 2): divides every group's N/16
+    const GemmTileSet* sets = nullptr;  // the workgroups' tiles
     int num_sets = 0;
-    bool narrow = false;  // prefer 64-column waves to 128-column ones (long K)
 };
 
 // Readout batches: up to kReadoutBatch receivers of one type, as a range of
@@ -337,8 +338,11 @@ void set_last_error(const std::string& message);
 std::unique_ptr<KernelSet> make_kernel_set(int C, int l_max, int L_max, const std::vector<std::int32_t>& m0_terms,
                                            const std::vector<std::int32_t>& m0_offsets,
                                            const std::vector<std::int32_t>& m1_terms);
-// [K][N] row-major block -> MFMA B-operand order [K/16][N/16][4][16][4]
-// (k chunk, column block, lane/16, lane%16, k within the lane's four)
+// count row-major [K][N] blocks (device) -> the GEMM's operand order
+// [K/32][N/16][3 parts][64 lanes][8] bf16 of each (device, 6 bytes a weight)
+void launch_pack_gemm_weights(const float* w, std::size_t count, int K, int N, void* out, hipStream_t s);
+// one row-major [K][N] block -> FP32 order [K/16][N/16][4][16][4] of the
+// one-wave form (k chunk, column block, lane/16, lane%16, k within the lane's four)
 void swizzle_gemm_weights(const float* w, int K, int N, float* out);
 // paths of the compiled kernel set for (l_max, L_max), false if none
 bool kernel_paths(int l_max, int L_max, std::vector<int>& le, std::vector<int>& ls, std::vector<int>& lo);
@@ -361,7 +365,7 @@ void geometry_records(int l_max, std::int64_t E, const double* xyz, const double
 void launch_edge_pairs(std::int64_t E, const int* receivers, const int* node_types, const int* neigh_types,
                        const int* type_to_active, int active_types, int* edge_pair, int* bad, hipStream_t s);
 
-void launch_node_gemm(const GemmPlan& plan, const float* W, const float* in, float* out, hipStream_t s);
+void launch_node_gemm(const GemmPlan& plan, const GemmWeights& W, const float* in, float* out, hipStream_t s);
 // rows[li][0..row_len) += bias[types[r0 + li]][0..row_len) for li < nr
 void launch_type_bias(int r0, int nr, const int* types, int row_len, const float* bias, float* rows, hipStream_t s);
 
