@@ -2,8 +2,9 @@
 """Checks this library's gfx950 assembly for MFMA results read too early.
 
 An instruction that reads a register written by v_mfma_f32_16x16x4_f32 (8
-passes) must issue at least ten wait states after it, on every path; the
-hardware does not interlock.  The compiler inserts the waits, but in kernels
+passes) must issue at least ten wait states after it, on every path, and one
+that touches a register written by v_mfma_f32_16x16x32_bf16 (4 passes) at least
+eight; the hardware does not interlock.  The compiler inserts the waits, but in kernels
 whose MFMA chains sat in runtime-conditional blocks it padded only the
 fall-through path into a join, and a read on the taken branch came one
 instruction after its MFMA (a stale accumulator element, silently wrong).
@@ -26,6 +27,10 @@ from collections import defaultdict
 _BRANCH = re.compile(r"s_(?:c?branch\w*)\s+(\.LBB\w+)")
 _RANGE = re.compile(r"([av])\[(\d+):(\d+)\]$")
 _SINGLE = re.compile(r"([av])(\d+)$")
+
+
+# wait states an MFMA asks for less than the default (16x16x4 FP32, 8 passes)
+_SLACK = {"v_mfma_f32_16x16x32_bf16": 2}  # 4 passes
 
 
 def _regs(token):
@@ -98,7 +103,7 @@ def findings(body, minimum):
         for k in range(idx - 1, -1, -1):
             t = ins[k]
             if t.startswith("v_mfma") and reg in _regs(t.split(None, 1)[1].split(",")[0]):
-                return d
+                return d + _SLACK.get(t.split()[0], 0)
             d += _cost(t)
             if d >= budget:
                 return budget
@@ -117,7 +122,7 @@ def findings(body, minimum):
             for op in (ops[1:] if t.startswith("v_") else ops):
                 for reg in _regs(op):
                     d = since_mfma(bi, k, reg, minimum, frozenset())
-                    if d < minimum:
+                    if d < minimum:  # (a bf16 MFMA's distance counts its slack)
                         out.append((b["label"], t, "%s%d" % reg, d))
     return out
 

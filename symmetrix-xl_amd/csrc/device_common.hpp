@@ -88,6 +88,50 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
+// FP32 matrix products on bf16 MFMAs: an FP32 value as three bf16 parts, each
+// the rounding of what the ones before it left.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+
+struct SplitOperand {
+    bf16x8 part[3];
+};
+
+// (pairs by hand: one v_cvt_pk_bf16_f32 rounds two values, and a part's value
+// is its bits in the upper half)
+__device__ __forceinline__ SplitOperand split_operand(f32x8 x) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    SplitOperand o;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        u32x4 bits;
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            const f32x2 v = {x[2 * h], x[2 * h + 1]};
+            bits[h] = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+            if (p < 2) {
+                x[2 * h] -= __uint_as_float(bits[h] << 16);
+                x[2 * h + 1] -= __uint_as_float(bits[h] & 0xffff0000u);
+            }
+        }
+        o.part[p] = __builtin_bit_cast(bf16x8, bits);
+    }
+    return o;
+}
+
+// acc + a b over 32 channels (v_mfma_f32_16x16x32_bf16) from the parts, the
+// smallest products first; the products left out are below 2^-26 |a b|.
+typedef float acc4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ acc4 split_product(const SplitOperand& a, const SplitOperand& b, acc4 acc) {
+    constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.part[pa[q]], b.part[pb[q]], acc, 0, 0, 0);
+    return acc;
+}
+
 inline unsigned blocks_for(std::int64_t n, int per_block) {
     return static_cast<unsigned>((n + per_block - 1) / per_block);
 }

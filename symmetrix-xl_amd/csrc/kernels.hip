@@ -1034,48 +1034,13 @@ __global__ void k_fill_f64(std::size_t n, double* __restrict__ p) {
 // contiguous bytes a row) and holds columns 4*(l/16).. +3 of row l%16.  Rows
 // past the set's count repeat its last row and store nothing.
 // ---------------------------------------------------------------------------
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-
-struct SplitOperand {
-    bf16x8 part[3];
-};
-
-// (pairs by hand: one v_cvt_pk_bf16_f32 rounds two values, and a part's value
-// is its bits in the upper half)
-__device__ __forceinline__ SplitOperand split_operand(f32x8 x) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    SplitOperand o;
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-        u32x4 bits;
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-            const f32x2 v = {x[2 * h], x[2 * h + 1]};
-            bits[h] = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
-            if (p < 2) {
-                x[2 * h] -= __uint_as_float(bits[h] << 16);
-                x[2 * h + 1] -= __uint_as_float(bits[h] & 0xffff0000u);
-            }
-        }
-        o.part[p] = __builtin_bit_cast(bf16x8, bits);
-    }
-    return o;
-}
-
 // acc[i] += (a[i] b)^T from the parts, the smallest products first.  The
 // weights are the MFMA's A operand, so a lane ends with four consecutive
 // columns of its row and stores them with 16 bytes.
 template <int RT>
 __device__ __forceinline__ void split_mfma(const SplitOperand (&a)[RT], const SplitOperand& b, v4f (&acc)[RT]) {
-    constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-    for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int q = 0; q < 6; ++q)
-            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.part[pb[q]], a[i].part[pa[q]], acc[i], 0, 0, 0);
+    for (int i = 0; i < RT; ++i) acc[i] = split_product(b, a[i], acc[i]);
 }
 
 // One thread per (chunk, 16-column block, lane): its eight weights in three

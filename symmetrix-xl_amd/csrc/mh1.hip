@@ -80,6 +80,7 @@ constexpr int kRegTilesFwd = 2, kRegTilesRev = 1, kRegTilesOut = 2;
 struct DMlpStage {
     int in, out, w, b, wt, ln;
     float eps;
+    int pw, pwt;  // parts of W and W^T (pack_parts), in 16-byte units of DMlp::parts
 };
 
 struct DMlp {
@@ -92,6 +93,7 @@ struct DMlp {
     const int* tape_offset;  // per layer: output offset in the edge's tape row (-1: last layer)
     int reg_hw, reg_stages;  // register form (reg_hw 0: the LDS-tile kernels run)
     DMlpStage st[kRegStages + 1];  // hidden stages from 0, the final linear at kRegStages
+    const bf16x8* parts;
 };
 
 // the reverse of a register-form MLP with a wide final linear runs in two kernels
@@ -623,15 +625,23 @@ __global__ __launch_bounds__(256) void k_mlp_reverse(const DMlp m, const DRadial
 // ---- edge MLPs in registers
 //
 // The units of a layer are the rows and the edges the columns of
-// v_mfma_f32_16x16x4_f32: lane (r, kg) of a wave (r = lane % 16, kg =
-// lane / 16) holds, for edge e0 + 16t + r of its t-th tile of 16 edges,
-// units 16i + 4kg + v (v < 4) of a layer in x[t][i][v] (the D layout).  With
-// the k index of step (J, v) of lane group kg taken as 16J + 4kg + v, the same
-// registers are the B operand of the next layer, and the A operand (weight row
-// 16i + r) is one 16-byte load per J: a tile's activations never leave
+// v_mfma_f32_16x16x32_bf16 over bf16 parts (split_product): lane (r, kg) of a
+// wave (r = lane % 16, kg = lane / 16) holds, for edge e0 + 16t + r of its t-th
+// tile of 16 edges, units 16i + 4kg + v (v < 4) of a layer in x[t][i][v] (the D
+// layout).  With channels 32c + 4kg + v and 32c + 16 + 4kg + v as lane group
+// kg's eight of chunk c, the same registers, split, are the B operand of the
+// next layer; the A operand (weight row 16i + r, split when the model is
+// loaded) is one 16-byte load per part: a tile's activations never leave
 // registers and no LDS is used.  Every hidden stage has the width 16 MT, so
 // the MFMA chains are straight-line code.  Lanes r, r+16, r+32, r+48 hold one edge, so
 // a LayerNorm's row sums are the lane's 16 units plus two cross-group shuffles.
+// In FP32 products (v_mfma_f32_16x16x4_f32) the MFMAs were the larger half of
+// these kernels' issue time; the parts' six MFMAs take 96 cycles for 32
+// channels where the FP32 form takes 256, and split the activations with 44
+// VALU instructions an edge tile and chunk.  At 184,320 edges (40-64-64-64-128
+// and -320): forward 338 -> 224 us, output reverse 202 -> 158, reverse 351 ->
+// 252.  What is left is LayerNorm and SiLU, the weights' way through L1 (138 KB
+// a 16-edge tile in the reverse) and, for the wide outputs, HBM.
 // The reverse recomputes the hidden stages from the radial features instead
 // of reading a tape, as the reference's streamed reverse re-runs the
 // conditioned MLPs per edge block (mace_nonlinear.cpp:916-929).
@@ -672,30 +682,44 @@ __device__ __forceinline__ float group4_sum(float v) {
     return v;
 }
 
-// acc[t][i] = sum_k W[16i + r][k] x[t][k] (W row-major with row stride K; K = M = 16 MT)
+// weights of chunk c and rows 16i.. +15 of a packed matrix of nblk 16-row blocks
+__device__ __forceinline__ SplitOperand ld_parts(const bf16x8* __restrict__ parts, int off, int nblk, int c, int i) {
+    const bf16x8* p = parts + off + (c * nblk + i) * 192 + (threadIdx.x & 63);
+    return SplitOperand{{p[0], p[64], p[128]}};
+}
+
+// a lane's units of two 16-unit blocks (zeros for the second one of the last odd block) as chunk c's operand
+template <int MT>
+__device__ __forceinline__ SplitOperand reg_split(const float (&x)[MT][4], int c) {
+    f32x8 v{};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        v[q] = x[2 * c][q];
+        if (2 * c + 1 < MT) v[4 + q] = x[2 * c + 1 < MT ? 2 * c + 1 : 0][q];
+    }
+    return split_operand(v);
+}
+
+// acc[t][i] = sum_k W[16i + r][k] x[t][k] (W packed at `off`; K = M = 16 MT)
 template <int MT, int NT>
-__device__ __forceinline__ void reg_linear(const float* __restrict__ W, int K, int M, const float (&x)[NT][MT][4],
+__device__ __forceinline__ void reg_linear(const bf16x8* __restrict__ parts, int off, const float (&x)[NT][MT][4],
                                            v4f (&acc)[NT][MT]) {
-    const int lane = threadIdx.x & 63, r = lane & 15, kg = lane >> 4;
+    constexpr int NC = (MT + 1) / 2;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[t][i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int J = 0; J < MT; ++J) {
-        v4f a[MT];
+    for (int c = 0; c < NC; ++c) {
+        SplitOperand b[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) b[t] = reg_split<MT>(x[t], c);
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-            a[i] = ld4(W + static_cast<std::size_t>(16 * i + r) * K + 16 * J + 4 * kg);
+            const SplitOperand a = ld_parts(parts, off, MT, c, i);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[t][i] = split_product(a, b[t], acc[t][i]);
         }
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-#pragma unroll
-            for (int i = 0; i < MT; ++i) {
-#pragma unroll
-                for (int t = 0; t < NT; ++t)
-                    acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][v], x[t][J][v], acc[t][i], 0, 0, 0);
-            }
     }
     mfma_settle();
 }
@@ -806,21 +830,19 @@ __device__ __forceinline__ void reg_hidden(const DMlp& m, long long E, long long
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[t][i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     const DMlpStage& S0 = m.st[0];
-    const float* W0 = m.params + S0.w;  // [S0.out][nb]
-    for (int k0 = 0; k0 < nb; k0 += 4) {
-        const int k = k0 + kg;
-        float b[NT];
+    for (int c = 0; 32 * c < nb; ++c) {
+        SplitOperand b[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            b[t] = 0.0f;
-            if (k < nb) b[t] = rad[ec[t] * nb + k];
+            const float* row = rad + ec[t] * nb;
+            const v4f lo = ld4_row(row, 32 * c + 4 * kg, nb), hi = ld4_row(row, 32 * c + 16 + 4 * kg, nb);
+            b[t] = split_operand(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         }
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-            float a = 0.0f;
-            if (k < nb) a = W0[(16 * i + r) * nb + k];
+            const SplitOperand a = ld_parts(m.parts, S0.pw, MT, c, i);
 #pragma unroll
-            for (int t = 0; t < NT; ++t) acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b[t], acc[t][i], 0, 0, 0);
+            for (int t = 0; t < NT; ++t) acc[t][i] = split_product(a, b[t], acc[t][i]);
         }
     }
     mfma_settle();
@@ -838,7 +860,7 @@ __device__ __forceinline__ void reg_hidden(const DMlp& m, long long E, long long
     for (int h = 1; h < kRegStages; ++h) {
         if (h >= m.reg_stages) break;
         const DMlpStage& S = m.st[h];
-        reg_linear<MT, NT>(m.params + S.w, S.in, S.out, x, acc);
+        reg_linear<MT, NT>(m.parts, S.pw, x, acc);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -861,27 +883,29 @@ __global__ __launch_bounds__(256) void k_mlp_forward_r(const DMlp m, long long E
     float x[NT][MT][4], xs[kRegStages][NT][MT][4], rs[kRegStages][NT];
     reg_hidden<HW, NT, false>(m, E, e0, rad, ets, ett, x, xs, rs);
     const DMlpStage& F = m.st[kRegStages];
-    const float* W = m.params + F.w;
     const float* bias = m.params + F.b;
-    const int K = F.in, M = F.out;
-    // two 16-row tiles of the output per pass (independent MFMA chains); rows past M read row M-1
-    // and are not stored
+    const int M = F.out, nblk = (M + 15) / 16;
+    constexpr int NC = (MT + 1) / 2;
+    SplitOperand b[NT][NC];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) b[t][c] = reg_split<MT>(x[t], c);
+    // two 16-row tiles of the output per pass (independent MFMA chains); rows past M have zero
+    // weights (or, a whole tile of them, the last tile's) and are not stored
     for (int i0 = 0; i0 < M; i0 += 32) {
-        const int ra = min(i0 + r, M - 1), rb = min(i0 + 16 + r, M - 1);
+        const int ia = i0 / 16, ib = min(ia + 1, nblk - 1);
         v4f acc[NT][2];
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t][0] = acc[t][1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int J = 0; J < MT; ++J) {
-                const v4f a0 = ld4(W + static_cast<std::size_t>(ra) * K + 16 * J + 4 * kg);
-            const v4f a1 = ld4(W + static_cast<std::size_t>(rb) * K + 16 * J + 4 * kg);
+        for (int c = 0; c < NC; ++c) {
+            const SplitOperand a0 = ld_parts(m.parts, F.pw, nblk, c, ia), a1 = ld_parts(m.parts, F.pw, nblk, c, ib);
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[v], x[t][J][v], acc[t][0], 0, 0, 0);
-                    acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[v], x[t][J][v], acc[t][1], 0, 0, 0);
-                }
+            for (int t = 0; t < NT; ++t) {
+                acc[t][0] = split_product(a0, b[t][c], acc[t][0]);
+                acc[t][1] = split_product(a1, b[t][c], acc[t][1]);
+            }
         }
         mfma_settle();
         const v4f b0 = ld4_row(bias, i0 + 4 * kg, M), b1 = ld4_row(bias, i0 + 16 + 4 * kg, M);
@@ -897,31 +921,30 @@ __global__ __launch_bounds__(256) void k_mlp_forward_r(const DMlp m, long long E
 }
 
 // Adjoint of the last hidden stage's output from the final linear's output adjoint:
-// g[t][i] = sum_k W_F[k][16i + r] gout[e][k] (W_F^T rows as the A operand, gout rows as B).
+// g[t][i] = sum_k W_F[k][16i + r] gout[e][k] (packed W_F^T rows as the A operand, gout rows as B).
 template <int MT, int NT>
 __device__ __forceinline__ void reg_out_reverse(const DMlp& m, const long long (&ec)[NT], const float* __restrict__ gout,
                                                 v4f (&g)[NT][MT]) {
-    const int lane = threadIdx.x & 63, r = lane & 15, kg = lane >> 4;
+    const int kg = (threadIdx.x & 63) >> 4;
     const DMlpStage& F = m.st[kRegStages];
-    const float* WT = m.params + F.wt;  // [F.in][F.out]
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < MT; ++i) g[t][i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k0 = 0; k0 < F.out; k0 += 16) {
-        v4f gb[NT], a[MT];
+    for (int c = 0; 32 * c < F.out; ++c) {
+        SplitOperand b[NT];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) gb[t] = ld4_row(gout + ec[t] * F.out, k0 + 4 * kg, F.out);
+        for (int t = 0; t < NT; ++t) {
+            const float* row = gout + ec[t] * F.out;
+            const v4f lo = ld4_row(row, 32 * c + 4 * kg, F.out), hi = ld4_row(row, 32 * c + 16 + 4 * kg, F.out);
+            b[t] = split_operand(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
-            a[i] = ld4_row(WT + static_cast<std::size_t>(16 * i + r) * F.out, k0 + 4 * kg, F.out);
+        for (int i = 0; i < MT; ++i) {
+            const SplitOperand a = ld_parts(m.parts, F.pwt, MT, c, i);
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int t = 0; t < NT; ++t)
-                    g[t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][v], gb[t][v], g[t][i], 0, 0, 0);
+            for (int t = 0; t < NT; ++t) g[t][i] = split_product(a, b[t], g[t][i]);
+        }
     }
     mfma_settle();
 }
@@ -984,27 +1007,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         reg_silu_norm_reverse<MT, NT>(m.params, S, g, xs[h], rs[h], gx);
         if (h > 0) {
             // adjoint of the previous stage's output: W_h^T gx, W_h^T = [S.in][S.out] row-major
-            reg_linear<MT, NT>(m.params + S.wt, S.out, S.in, gx, g);
+            reg_linear<MT, NT>(m.parts, S.pwt, gx, g);
             continue;
         }
         // radial adjoint: rad_adj[e][k] += sum_u W0[u][k] gx[e][u], W0^T = [nb][S.out]
         const int nb = m.radial;
-        const float* WT0 = m.params + S.wt;
+        constexpr int NC = (MT + 1) / 2;
+        SplitOperand b[NT][NC];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) b[t][c] = reg_split<MT>(gx[t], c);
         for (int k0 = 0; k0 < nb; k0 += 16) {
-            const int kr = min(k0 + r, nb - 1);
-            const bool kv = k0 + r < nb;
             v4f acc[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int J = 0; J < MT; ++J) {
-                v4f a = ld4(WT0 + static_cast<std::size_t>(kr) * S.out + 16 * J + 4 * kg);
-                if (!kv) a = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int c = 0; c < NC; ++c) {
+                const SplitOperand a = ld_parts(m.parts, S.pwt, (nb + 15) / 16, c, k0 / 16);
 #pragma unroll
-                for (int v = 0; v < 4; ++v)
-#pragma unroll
-                    for (int t = 0; t < NT; ++t)
-                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[v], gx[t][J][v], acc[t], 0, 0, 0);
+                for (int t = 0; t < NT; ++t) acc[t] = split_product(a, b[t][c], acc[t]);
             }
             mfma_settle();
 #pragma unroll
@@ -1814,6 +1836,34 @@ struct Packer {
     }
 };
 
+// A row-major [M][K] matrix in the A-operand order of split_product: three bf16
+// parts of each weight (split_operand's), [K/32][M/16][3][64 lanes][8], both
+// padded with zeros.  Appends to out and returns the offset in 16-byte units.
+int pack_parts(const float* W, int M, int K, std::vector<std::uint16_t>& out) {
+    const std::size_t at = out.size();
+    const int chunks = (K + 31) / 32, nblk = (M + 15) / 16;
+    out.resize(at + static_cast<std::size_t>(chunks) * nblk * 3 * 64 * 8, 0);
+    for (int c = 0; c < chunks; ++c)
+        for (int i = 0; i < nblk; ++i)
+            for (int lane = 0; lane < 64; ++lane)
+                for (int e = 0; e < 8; ++e) {
+                    const int row = 16 * i + lane % 16, k = 32 * c + 4 * (lane / 16) + e % 4 + 16 * (e / 4);
+                    if (row >= M || k >= K) continue;
+                    float x = W[static_cast<std::size_t>(row) * K + k];
+                    for (int p = 0; p < 3; ++p) {
+                        std::uint32_t u;
+                        std::memcpy(&u, &x, 4);
+                        u = (u + 0x7fffu + (u >> 16 & 1u)) & 0xffff0000u;  // nearest, ties to even
+                        float part;
+                        std::memcpy(&part, &u, 4);
+                        out[at + ((((static_cast<std::size_t>(c) * nblk + i) * 3 + p) * 64 + lane) * 8) + e] =
+                            static_cast<std::uint16_t>(u >> 16);
+                        x -= part;
+                    }
+                }
+    return static_cast<int>(at / 8);
+}
+
 void Evaluator::upload_model() {
     Packer pk;
     struct LinOff {
@@ -1828,11 +1878,19 @@ void Evaluator::upload_model() {
                       !T.in_mask.empty(), T.in_dim, T.out_dim, T.out_blocks};
     };
     struct MlpOff {
-        std::size_t layers, eps, params, rows, wt, tape;
+        std::size_t layers, eps, params, rows, wt, tape, parts;
+        std::vector<int> pw;  // per stage: parts of W and W^T
     };
     auto put_mlp = [&](const MlpTables& T) {
-        return MlpOff{pk.put(T.layers), pk.put(T.eps), pk.put(T.params), pk.put(T.type_rows), pk.put(T.wt_offset),
-                      pk.put(T.tape_offset)};
+        std::vector<std::uint16_t> parts;
+        std::vector<int> pw;
+        for (int k = 0; T.reg_hw && k <= T.reg_stages; ++k) {
+            const int* S = &T.reg_stage[6 * k];
+            pw.push_back(pack_parts(T.params.data() + S[2], S[1], S[0], parts));
+            pw.push_back(pack_parts(T.params.data() + S[4], S[0], S[1], parts));
+        }
+        return MlpOff{pk.put(T.layers),    pk.put(T.eps),         pk.put(T.params), pk.put(T.type_rows),
+                      pk.put(T.wt_offset), pk.put(T.tape_offset), pk.put(parts),    pw};
     };
     const Model& M = model_;
     const int nt = static_cast<int>(M.atomic_numbers.size());
@@ -1951,11 +2009,13 @@ void Evaluator::upload_model() {
     };
     auto mlp = [&](const MlpTables& T, const MlpOff& o) {
         DMlp d{T.num_layers, T.radial, T.first_width, nt, T.max_hidden, T.tape_width, I_(o.layers), F(o.eps),
-               F(o.params), F(o.rows), I_(o.wt), I_(o.tape), T.reg_hw, T.reg_stages, {}};
+               F(o.params), F(o.rows), I_(o.wt), I_(o.tape), T.reg_hw, T.reg_stages, {},
+               reinterpret_cast<const bf16x8*>(base + o.parts)};
         // hidden stages from slot 0, the final linear in slot kRegStages
         for (int k = 0; T.reg_hw && k <= T.reg_stages; ++k) {
             const int* S = &T.reg_stage[6 * k];
-            d.st[k < T.reg_stages ? k : kRegStages] = DMlpStage{S[0], S[1], S[2], S[3], S[4], S[5], T.reg_eps[k]};
+            d.st[k < T.reg_stages ? k : kRegStages] = 
+                DMlpStage{S[0], S[1], S[2], S[3], S[4], S[5], T.reg_eps[k], o.pw[2 * k], o.pw[2 * k + 1]};
         }
         return d;
     };

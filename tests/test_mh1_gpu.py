@@ -328,3 +328,26 @@ def test_mh1_benchmark_size_rotation_and_translation(paths):
     assert abs(e1.sum() - e0.sum()) / len(e0) < 1e-5
     assert np.abs(e1 - e0).max() < 5e-4
     assert np.abs(F1 - F0 @ R.T).max() < 1e-4
+
+
+@pytest.mark.parametrize("name", ["mh1_tiny", "mh1_tiny_mlp32", "mh1_medium"])
+@pytest.mark.parametrize("n", [2, 3, 5, 6, 9])
+def test_mh1_edge_mlp_at_tile_edges(paths, name, n):
+    """Edge MLP outputs and forces of few edges (2, 6, 20, 30, 72: parts of a
+    16-edge tile, whole tiles and a remainder).  Bound of a weight: each of at
+    most four linears rounds a sum of at most 64 terms in FP32, 64 * 2^-24 of
+    its scale."""
+    model = mo.MH1Oracle(paths[name])
+    rng = np.random.default_rng(n)
+    sites = np.stack(np.meshgrid(*(np.arange(3),) * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    pos = sites * 1.4 + rng.uniform(-0.1, 0.1, size=(n, 3))
+    cell = np.eye(3) * 30.0
+    types = rng.integers(0, len(model.atomic_numbers), size=n).astype(np.int32)
+    g, xyz, r = _graph(model, pos, cell)
+    _, f_ref = model.evaluate(types, g["receivers"], g["sources"], xyz)
+    ev, _, f = _gpu(paths[name], types, g, xyz, r)
+    for k, state in enumerate(model.stages["states"]):
+        ref = np.asarray(state["wraw"])
+        got = ev._stage("w%d" % k).reshape(ref.shape)
+        assert np.abs(got - ref).max() <= 4 * 64 * 2.0 ** -24 * max(1.0, np.abs(ref).max())
+    assert np.abs(f - f_ref).max() < 1e-4 * max(1.0, np.abs(f_ref).max())
