@@ -30,6 +30,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <limits>
 #include <map>
 #include <memory>
 #include <numeric>
@@ -2125,7 +2126,17 @@ void Evaluator::compute(int N, const int* types, const int* num_neigh, const int
         total += num_neigh[i];
     }
     if (total != E) throw std::invalid_argument("MH-1: neighbour counts do not sum to the edge count");
+    // whole-array passes without branches (the loop below finds which edge and why)
+    int bad = 0;
     for (long long e = 0; e < E; ++e) {
+        const unsigned src = static_cast<unsigned>(neigh[e]);
+        const bool in = src < static_cast<unsigned>(N);
+        bad |= !in | (neigh_types[e] != types[in ? src : 0]);
+    }
+    constexpr double kFinite = std::numeric_limits<double>::max();
+    for (long long e = 0; e < E; ++e) bad |= !(r[e] > 0.0) | !(r[e] <= kFinite);
+    for (long long q = 0; q < 3 * E; ++q) bad |= !(std::fabs(xyz[q]) <= kFinite);
+    for (long long e = 0; bad && e < E; ++e) {
         if (neigh[e] < 0 || neigh[e] >= N || neigh_types[e] != types[neigh[e]])
             throw std::invalid_argument("MH-1: edge source out of range or of the wrong type");
         if (!(r[e] > 0.0) || !std::isfinite(r[e]) || !std::isfinite(xyz[3 * e]) || !std::isfinite(xyz[3 * e + 1]) ||
@@ -2135,24 +2146,15 @@ void Evaluator::compute(int N, const int* types, const int* num_neigh, const int
     // past the checks a call replaces the results (a rejected graph leaves the last ones)
     num_energies_ = num_forces_ = 0;
     ensure_device();
-    // ---- host-side graph arrays
-    std::vector<int> offsets(N + 1, 0), tt(E), t_off(N + 1, 0), t_edges(E);
-    for (int i = 0; i < N; ++i) offsets[i + 1] = offsets[i] + num_neigh[i];
-    for (int i = 0; i < N; ++i)
-        for (int e = offsets[i]; e < offsets[i + 1]; ++e) tt[e] = types[i];
-    for (long long e = 0; e < E; ++e) ++t_off[neigh[e] + 1];
-    for (int i = 0; i < N; ++i) t_off[i + 1] += t_off[i];
-    {
-        std::vector<int> fill(t_off.begin(), t_off.end() - 1);
-        for (long long e = 0; e < E; ++e) t_edges[fill[neigh[e]]++] = static_cast<int>(e);
-    }
     const int NY = M.num_lm, R = static_cast<int>(M.bessel.size());
     const int L = static_cast<int>(M.interactions.size());
     // ---- workspace layout
     Layout lay;
-    const std::size_t o_types = lay.add<int>(N), o_off = lay.add<int>(N + 1), o_src = lay.add<int>(E),
-                      o_ts = lay.add<int>(E), o_tt = lay.add<int>(E), o_toff = lay.add<int>(N + 1),
-                      o_tedge = lay.add<int>(E), o_xyz = lay.add<double>(3 * E), o_r = lay.add<double>(E),
+    const std::size_t o_types = lay.add<int>(N), o_elems = lay.add<int>(N), o_off = lay.add<int>(N + 1),
+                      o_src = lay.add<int>(E), o_ts = lay.add<int>(E), o_tt = lay.add<int>(E),
+                      o_xyz = lay.add<double>(3 * E), o_r = lay.add<double>(E),
+                      // (the edges per source, which only the reverse reads)
+                      o_toff = lay.add<int>(N + 1), o_tedge = lay.add<int>(E),
                       o_Y = lay.add<float>(static_cast<std::size_t>(E) * NY), o_cut = lay.add<float>(E),
                       o_rad = lay.add<float>(static_cast<std::size_t>(E) * M.bessel.size()),
                       o_feat0 = lay.add<float>(static_cast<std::size_t>(N) * embed_dim_);
@@ -2199,7 +2201,6 @@ void Evaluator::compute(int N, const int* types, const int* num_neigh, const int
     for (const InteractionDev& I : inter_)
         for (const DMlp* m : {&I.wmlp, &I.dmlp})
             if (mlp_split(*m)) mlpg_width = std::max(mlpg_width, m->reg_hw);
-    const std::size_t o_elems = lay.add<int>(N);
     const std::size_t o_ro = lay.add<float>(static_cast<std::size_t>(L) * N),
                       o_h = lay.add<float>(static_cast<std::size_t>(N) * ro_width),
                       o_act = lay.add<float>(static_cast<std::size_t>(N) * ro_width),
@@ -2212,26 +2213,41 @@ void Evaluator::compute(int N, const int* types, const int* num_neigh, const int
     auto f = [&](std::size_t o) { return reinterpret_cast<float*>(W + o); };
     auto ip = [&](std::size_t o) { return reinterpret_cast<int*>(W + o); };
     auto dp = [&](std::size_t o) { return reinterpret_cast<double*>(W + o); };
-    // the host inputs lead the layout: staged at their device offsets in pinned memory, one transfer
-    const std::size_t in_end = o_r + sizeof(double) * static_cast<std::size_t>(E);
-    host_in_.reserve(in_end);
+    // The host inputs lead the layout: formed at their device offsets in pinned
+    // memory.  What the forward reads goes in one transfer; the edges per
+    // source are formed while the device runs the forward.
+    const std::size_t in_end = o_r + sizeof(double) * static_cast<std::size_t>(E),
+                      in_end2 = o_tedge + sizeof(int) * static_cast<std::size_t>(E);
+    host_in_.reserve(in_end2);
     char* H = host_in_.base();
     auto put = [&](std::size_t o, const void* src, std::size_t bytes) {
         if (bytes) std::memcpy(H + o, src, bytes);
     };
+    auto hi = [&](std::size_t o) { return reinterpret_cast<int*>(H + o); };
+    std::vector<int> fill(N);
     put(o_types, types, sizeof(int) * N);
-    put(o_off, offsets.data(), sizeof(int) * (N + 1));
     put(o_src, neigh, sizeof(int) * E);
     put(o_ts, neigh_types, sizeof(int) * E);
-    put(o_tt, tt.data(), sizeof(int) * E);
-    put(o_toff, t_off.data(), sizeof(int) * (N + 1));
-    put(o_tedge, t_edges.data(), sizeof(int) * E);
     put(o_xyz, xyz, sizeof(double) * 3 * E);
     put(o_r, r, sizeof(double) * E);
+    hi(o_off)[0] = 0;
+    for (int i = 0, e = 0; i < N; ++i) {
+        hi(o_elems)[i] = M.model_indices[types[i]];
+        std::fill_n(hi(o_tt) + e, num_neigh[i], types[i]);
+        hi(o_off)[i + 1] = e += num_neigh[i];
+    }
     SMX_HIP(hipMemcpyAsync(W, H, in_end, hipMemcpyHostToDevice, stream_));
-    std::vector<int> midx(N);
-    for (int i = 0; i < N; ++i) midx[i] = M.model_indices[types[i]];
-    if (N) SMX_HIP(hipMemcpyAsync(W + o_elems, midx.data(), sizeof(int) * N, hipMemcpyHostToDevice, stream_));
+    auto send_sources = [&] {
+        int *t_off = hi(o_toff), *t_edges = hi(o_tedge);
+        std::fill_n(t_off, N + 1, 0);
+        for (long long e = 0; e < E; ++e) ++t_off[neigh[e] + 1];
+        for (int i = 0; i < N; ++i) {
+            fill[i] = t_off[i];
+            t_off[i + 1] += t_off[i];
+        }
+        for (long long e = 0; e < E; ++e) t_edges[fill[neigh[e]]++] = static_cast<int>(e);
+        SMX_HIP(hipMemcpyAsync(W + o_toff, H + o_toff, in_end2 - o_toff, hipMemcpyHostToDevice, stream_));
+    };
     const int* d_types = ip(o_types);
     const int* d_off = ip(o_off);
     const int* d_src = ip(o_src);
@@ -2346,6 +2362,7 @@ void Evaluator::compute(int N, const int* types, const int* num_neigh, const int
     }
     launch("mh1_energies", k_energies, blocks_for(N, 256), 256, 0, N, L, d_types, atomic_e_, M.scale, M.shift, ro,
            d_off, d_ts, d_r, zbl_, M.has_zbl ? 1 : 0, dp(o_en));
+    send_sources();
     // ---- reverse (mace_nonlinear.cpp:782-1000)
     const float scale_f = static_cast<float>(M.scale);
     launch("mh1_fill", k_fill, blocks_for(N, 256), 256, 0, static_cast<long long>(N), scale_f, f(o_ones));
