@@ -1927,7 +1927,7 @@ void launch_node_gemm(const GemmPlan& plan, const GemmWeights& W, const float* i
             plan.sets, plan.groups, plan.rows, static_cast<const bf16x8*>(W.packed), in, out);
     };
     // Few rows: the wave form until 64-column workgroups would give every CU
-    // one (the six linears of 320 medium-model nodes 44 us in it; a workgroup
+    // two (the six linears of 320 medium-model nodes 44 us in it; a workgroup
     // form's launch takes about 10 us at any number of rows below, a wave
     // form's 5 to 10).  Above, 128 columns a workgroup once that gives each CU two of them,
     // else 64 (128 x 128 with the launch's 5.9 us: 20,000 rows 14.0 against

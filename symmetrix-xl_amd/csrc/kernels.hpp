@@ -137,9 +137,9 @@ struct GemmGroup {
 // kernel, rows [row_start, row_start+count) of the plan's row list.
 constexpr int kGemmSetTiles = 8;
 constexpr int kGemmSetRows = 16 * kGemmSetTiles;
-// workgroups from which a launch takes the workgroup form (one per CU), and
+// workgroups from which a launch takes the workgroup form (two per CU), and
 // from which their column blocks widen (two per CU)
-constexpr long long kGemmWaveFill = 256, kGemmFill = 512;
+constexpr long long kGemmWaveFill = 512, kGemmFill = 512;
 struct GemmTileSet {
     int row_start, count, group;
 };
