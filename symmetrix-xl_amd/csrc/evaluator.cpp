@@ -188,13 +188,22 @@ private:
     std::vector<std::string> order_;
 };
 
-// Concatenated node-linear rows and sets of every receiver tile of the graph.
+// Concatenated node-linear tiles of every receiver tile of the graph.
 struct PlanSet {
-    std::vector<int> rows;          // packed (local node << 4 | m)
-    std::vector<GemmTileSet> sets;
-    std::vector<std::size_t> set_begin;  // per receiver tile: its first set
-    DevBuf d_rows, d_sets;
+    std::vector<GemmTile> tiles;
+    std::vector<std::size_t> tile_begin;  // per receiver tile: first GemmTile
+    std::vector<int> rows;                // packed (local node << 4 | m)
+    std::vector<GemmTileSet> sets;        // per receiver tile, tiles relative to its first
+    std::vector<std::size_t> set_begin;
+    DevBuf d_tiles, d_rows, d_sets;
 };
+
+// the set of tiles [t, min(t + kGemmShareWaves, t1)), counted from `base`
+GemmTileSet gemm_set(const std::vector<GemmTile>& tiles, std::size_t base, int t, int t1) {
+    const int n = std::min(kGemmShareWaves, t1 - t);
+    const GemmTile &a = tiles[base + t], &b = tiles[base + t + n - 1];
+    return GemmTileSet{t, n, a.row_start, b.row_start + b.count - a.row_start, a.group};
+}
 
 }  // namespace
 
@@ -525,21 +534,29 @@ struct Evaluator {
         std::size_t count;
         int K, N;
     };
-    // a weight array on the device in the GEMM kernels' operand orders
+    // a weight array on the device in the operand order of the form that the
+    // model's node linears run in (kGemmPartsChannels)
     GemmWeights put_gemm(const std::vector<float>& w, const std::vector<GemmBlocks>& blocks) {
-        DevBuf raw;
-        const float* src = upload(raw, w, stream);
-        model_bufs.push_back(std::make_unique<DevBuf>());
-        char* dst = static_cast<char*>(model_bufs.back()->ensure(std::max<std::size_t>(1, w.size()) * 6));
-        std::vector<float> waves(w.size());
-        for (const auto& b : blocks) {
-            launch_pack_gemm_weights(src + b.first, b.count, b.K, b.N, dst + 6 * b.first, stream);
-            const std::size_t blk = static_cast<std::size_t>(b.K) * b.N;
-            for (std::size_t q = 0; q < b.count; ++q)
-                swizzle_gemm_weights(w.data() + b.first + q * blk, b.K, b.N, waves.data() + b.first + q * blk);
+        GemmWeights out;
+        if (hm.C >= kGemmPartsChannels) {
+            DevBuf raw;
+            const float* src = upload(raw, w, stream);
+            model_bufs.push_back(std::make_unique<DevBuf>());
+            char* dst = static_cast<char*>(model_bufs.back()->ensure(std::max<std::size_t>(1, w.size()) * 6));
+            for (const auto& b : blocks)
+                launch_pack_gemm_weights(src + b.first, b.count, b.K, b.N, dst + 6 * b.first, stream);
+            SMX_HIP(hipStreamSynchronize(stream));
+            out.parts = dst;
+        } else {
+            std::vector<float> waves(w.size());
+            for (const auto& b : blocks)
+                for (std::size_t q = 0; q < b.count; ++q) {
+                    const std::size_t at = b.first + q * static_cast<std::size_t>(b.K) * b.N;
+                    swizzle_gemm_weights(w.data() + at, b.K, b.N, waves.data() + at);
+                }
+            out.fp32 = put(waves);
         }
-        SMX_HIP(hipStreamSynchronize(stream));
-        return GemmWeights{dst, put(waves)};
+        return out;
     }
     GemmWeights put_gemm(const std::vector<float>& w, std::size_t count, int K, int N) {
         return put_gemm(w, {GemmBlocks{0, count, K, N}});
@@ -580,7 +597,7 @@ struct Evaluator {
         max_n_a1r = mx(groups_a1r);
         sub_a0 = sub(groups_a0);
         sub_h1 = sub(groups_h1);
-        sub_a1f = sub(groups_a1f);
+        sub_a1f = sub(groups_a1f);  // (the A1 forward plan prefers 64 columns: K runs to 3C)
         sub_a1r = sub(groups_a1r);
         upload(d_groups_a0, groups_a0, stream);
         upload(d_groups_h1, groups_h1, stream);
@@ -798,8 +815,10 @@ struct Evaluator {
     // one tile over all F feature nodes: the h1 (U, U^T), fz and fy plans
     void build_feature_tile() {
         for (PlanSet* p : {&ps_feat_h1, &ps_feat_fz, &ps_feat_fy}) {
+            p->tiles.clear();
             p->rows.clear();
             p->sets.clear();
+            p->tile_begin.assign(1, 0);
             p->set_begin.assign(1, 0);
         }
         auto add = [&](PlanSet& P, int group, int l) {
@@ -807,8 +826,12 @@ struct Evaluator {
             for (int m = 0; m < 2 * l + 1; ++m)
                 for (int q = 0; q < F; ++q) P.rows.push_back(q << 4 | m);
             const int end = static_cast<int>(P.rows.size());
-            for (int s0 = start; s0 < end; s0 += kGemmSetRows)
-                P.sets.push_back(GemmTileSet{s0, std::min(kGemmSetRows, end - s0), group});
+            const int t0 = static_cast<int>(P.tiles.size());
+            for (int s0 = start; s0 < end; s0 += kGemmRows)
+                P.tiles.push_back(GemmTile{s0, std::min(kGemmRows, end - s0), group});
+            const int t1 = static_cast<int>(P.tiles.size());
+            for (int t = t0; t < t1; t += kGemmShareWaves)
+                P.sets.push_back(gemm_set(P.tiles, 0, t, t1));
         };
         for (int l = 0; l <= hm.L_max; ++l) add(ps_feat_h1, l, l);
         for (std::size_t p = 0; p < hm.field_paths.size(); ++p) {
@@ -816,11 +839,15 @@ struct Evaluator {
             add(ps_feat_fy, static_cast<int>(p), hm.field_paths[p].l_out);
         }
         auto view = [&](PlanSet& P, const DevBuf& groups, int max_n, int n_sub) {
+            P.tile_begin.push_back(P.tiles.size());
             P.set_begin.push_back(P.sets.size());
+            upload(P.d_tiles, P.tiles, stream);
             upload(P.d_rows, P.rows, stream);
             upload(P.d_sets, P.sets, stream);
             GemmPlan g;
             g.n_sub = n_sub;
+            g.tiles = P.d_tiles.as<GemmTile>();
+            g.num_tiles = static_cast<int>(P.tiles.size());
             g.groups = groups.as<GemmGroup>();
             g.rows = P.d_rows.as<int>();
             g.max_n = max_n;
@@ -844,6 +871,8 @@ struct Evaluator {
         h_batches.clear();
         batch_begin.clear();
         for (PlanSet* p : {&ps_a0, &ps_h1, &ps_a1f, &ps_a1r, &ps_cap, &ps_fz, &ps_fy}) {
+            p->tiles.clear();
+            p->tile_begin.clear();
             p->rows.clear();
             p->sets.clear();
             p->set_begin.clear();
@@ -859,17 +888,22 @@ struct Evaluator {
             });
             h_node_list.insert(h_node_list.end(), order.begin(), order.end());
             for (PlanSet* p : {&ps_a0, &ps_h1, &ps_a1f, &ps_a1r, &ps_cap, &ps_fz, &ps_fy}) {
+                p->tile_begin.push_back(p->tiles.size());
                 p->set_begin.push_back(p->sets.size());
             }
             // rows (node order[a..b), m in [0, 2l+1)) of one group, cut into
-            // workgroups' sets
+            // wave tiles, and the tiles into sets of up to kGemmShareWaves
             auto add = [&](PlanSet& P, int group, int l, int a, int b) {
                 const int start = static_cast<int>(P.rows.size());
                 for (int m = 0; m < 2 * l + 1; ++m)
                     for (int q = a; q < b; ++q) P.rows.push_back(order[q] << 4 | m);
                 const int end = static_cast<int>(P.rows.size());
-                for (int s0 = start; s0 < end; s0 += kGemmSetRows)
-                    P.sets.push_back(GemmTileSet{s0, std::min(kGemmSetRows, end - s0), group});
+                const int t0 = static_cast<int>(P.tiles.size() - P.tile_begin.back());
+                for (int s0 = start; s0 < end; s0 += kGemmRows)
+                    P.tiles.push_back(GemmTile{s0, std::min(kGemmRows, end - s0), group});
+                const int t1 = static_cast<int>(P.tiles.size() - P.tile_begin.back());
+                for (int t = t0; t < t1; t += kGemmShareWaves)
+                    P.sets.push_back(gemm_set(P.tiles, P.tile_begin.back(), t, t1));
             };
             for (int p = 0; p < t.nr;) {
                 int q = p;
@@ -894,7 +928,9 @@ struct Evaluator {
         }
         batch_begin.push_back(h_batches.size());
         for (PlanSet* p : {&ps_a0, &ps_h1, &ps_a1f, &ps_a1r, &ps_cap, &ps_fz, &ps_fy}) {
+            p->tile_begin.push_back(p->tiles.size());
             p->set_begin.push_back(p->sets.size());
+            upload(p->d_tiles, p->tiles, stream);
             upload(p->d_rows, p->rows, stream);
             upload(p->d_sets, p->sets, stream);
         }
@@ -908,6 +944,8 @@ struct Evaluator {
         auto view = [&](const PlanSet& P, std::size_t ti, const DevBuf& groups, int max_n, int n_sub) {
             GemmPlan g;
             g.n_sub = n_sub;
+            g.tiles = P.d_tiles.as<GemmTile>() + P.tile_begin[ti];
+            g.num_tiles = static_cast<int>(P.tile_begin[ti + 1] - P.tile_begin[ti]);
             g.groups = groups.as<GemmGroup>();
             g.rows = P.d_rows.as<int>();
             g.max_n = max_n;
@@ -919,6 +957,7 @@ struct Evaluator {
             tiles[ti].a0 = view(ps_a0, ti, d_groups_a0, max_n_a0, sub_a0);
             tiles[ti].h1 = view(ps_h1, ti, d_groups_h1, max_n_h1, sub_h1);
             tiles[ti].a1f = view(ps_a1f, ti, d_groups_a1f, max_n_a1f, sub_a1f);
+            tiles[ti].a1f.narrow = true;
             tiles[ti].a1r = view(ps_a1r, ti, d_groups_a1r, max_n_a1r, sub_a1r);
             if (hm.pre_linear_up) {
                 tiles[ti].cap = view(ps_cap, ti, d_groups_cap, hm.C, sub_cap);
@@ -2354,6 +2393,17 @@ struct Evaluator {
     }
 
     std::int64_t stage(const std::string& name, float* out, std::int64_t capacity) {
+        if (name == "linear_forms") {  // (kind, columns, rows) of the first tile's A0, H1, A1 and A1 reverse linears
+            if (tiles.empty()) throw std::invalid_argument("stage 'linear_forms' needs a prepared graph");
+            const TileView& t = tiles[0];
+            int k = 0;
+            for (const GemmPlan* p : {&t.a0, &t.h1, &t.a1f, &t.a1r}) {
+                const NodeGemmForm f = node_gemm_form(*p, hm.C >= kGemmPartsChannels);
+                if (!out || capacity < 12) break;
+                for (int v : {f.kind, 16 * f.n_sub, 16 * f.tiles}) out[k++] = static_cast<float>(v);
+            }
+            return 12;
+        }
         const std::int64_t n = tiled ? max_tile_nr : N, C = hm.C, NY = hm.num_lm, NH = hm.num_LM,
                            NLME = hm.num_lme;
         const float* src = nullptr;

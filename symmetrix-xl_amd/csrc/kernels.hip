@@ -1009,31 +1009,217 @@ __global__ void k_fill_f64(std::size_t n, double* __restrict__ p) {
 }
 
 // ---------------------------------------------------------------------------
-// Node linears on MFMA, FP32 in and out, as products of bf16 parts
-// (v_mfma_f32_16x16x32_bf16 with FP32 accumulators): an FP32 value is the sum
-// of three bf16 values, each the rounding of what the ones before it left
-// (8 significand bits each, round to nearest, so 2^-27 of the value remains),
-// and x w = x1 w1 + x1 w2 + x2 w1 + x2 w2 + x1 w3 + x3 w1 up to 2^-26 |x w|,
-// below the 2^-24 of an FP32 product's own rounding.  Six such MFMAs cover
-// 32 input channels in 96 cycles where the FP32 form needs 256, and 24
-// accumulator updates instead of 32 round a sum of 128 terms.  (An input
-// beyond bf16's finite range, 3.39e38, or not finite gives NaN.)
-// Error of a 128-channel sum against 64 bits 1.5e-7 of its scale, 2.0e-7 in
-// FP32 products; all six linears of 5,000 medium-model nodes 177 us, 273 with
-// FP32 MFMAs; of 1,500 wide-model nodes 273 us, 435 before; 80,000 x 128 x 128
-// alone 20 us (4.1 TB/s of input and output), 41 before.
+// Node linears on MFMA (v_mfma_f32_16x16x4_f32, FP32 in and out).  One wave
+// computes a kGemmRows x 16*NSUB-column block as (kGemmRows/16) x NSUB tiles
+// of 16x16.  In a tile, lane l supplies A[l%16][kk] and B[kk][l%16] with
+// kk = l/16 and holds D[4*(l/16)+v][l%16].  The K order inside one 16-wide
+// chunk is permuted so that step s uses k = k0 + 4*(l/16) + s: each lane then
+// reads four consecutive inputs of its row with one 16-byte load, and the
+// weights are pre-swizzled (swizzle_gemm_weights) so that the B operands of
+// one chunk and 16-column block are one contiguous 1 KB float4 load per wave.
+// Per chunk a wave issues RI + NSUB loads and 4*RI*NSUB MFMAs.  Two operand
+// sets alternate: the loads of chunk kc+1 are in flight while chunk kc runs on
+// the MFMA unit (a three-set ring measured the same at the medium shape: it
+// costs two waves per SIMD of occupancy).  NSUB is a template constant so that the chunk body is
+// straight-line code (no per-tile branches) and the only waits are for the
+// operands of the chunk about to run.
+// ---------------------------------------------------------------------------
+template <int RI, int NSUB>
+struct GemmOperands {
+    float4 a[RI], b[NSUB];
+};
+
+template <int RI, int NSUB>
+__device__ __forceinline__ void gemm_load(GemmOperands<RI, NSUB>& o, const float* const (&arow)[RI],
+                                          const float4* __restrict__ B, int kc, int nblk) {
+#pragma unroll
+    for (int i = 0; i < RI; ++i) o.a[i] = *reinterpret_cast<const float4*>(arow[i] + 16 * kc);
+#pragma unroll
+    for (int j = 0; j < NSUB; ++j) o.b[j] = B[(static_cast<std::size_t>(kc) * nblk + j) * 64];
+}
+
+template <int RI, int NSUB>
+__device__ __forceinline__ void gemm_chunk(v4f (&acc)[RI][NSUB], const GemmOperands<RI, NSUB>& o) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+        for (int i = 0; i < RI; ++i) {
+            const float av = s == 0 ? o.a[i].x : s == 1 ? o.a[i].y : s == 2 ? o.a[i].z : o.a[i].w;
+#pragma unroll
+            for (int j = 0; j < NSUB; ++j) {
+                const float bv = s == 0 ? o.b[j].x : s == 1 ? o.b[j].y : s == 2 ? o.b[j].z : o.b[j].w;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc[i][j], 0, 0, 0);
+            }
+        }
+    }
+}
+
+template <int NSUB>
+__global__ __launch_bounds__(64) void k_node_gemm(const GemmTile* __restrict__ tiles,
+                                                  const GemmGroup* __restrict__ groups, const int* __restrict__ rows,
+                                                  const float* __restrict__ W, const float* __restrict__ in,
+                                                  float* __restrict__ out) {
+    constexpr int RI = kGemmRows / 16;  // 16-row MFMA tiles per wave
+    // blockIdx.x: row tile; blockIdx.y: 16*NSUB-column block.  (Dispatch
+    // order x-fastest: concurrent waves share one column block's weights.
+    // Grouping a tile's column blocks on one XCD measured slower.)
+    const GemmTile tile = tiles[blockIdx.x];
+    const GemmGroup g = groups[tile.group];
+    const int n0 = blockIdx.y * 16 * NSUB;
+    if (n0 >= g.N) return;
+    const int lane = threadIdx.x;
+    const int r = lane & 15, kg = lane >> 4;
+    const float* arow[RI];
+#pragma unroll
+    for (int i = 0; i < RI; ++i) {
+        // rows past the tile's count repeat its last row (their results are not stored)
+        const int q = min(16 * i + r, tile.count - 1);
+        const int pk = rows[tile.row_start + q];
+        arow[i] = in + static_cast<std::size_t>(pk >> 4) * g.in_stride + g.in_base + (pk & 15) * g.in_mstride + 4 * kg;
+    }
+    const int nblk = g.N / 16;
+    const float4* B = reinterpret_cast<const float4*>(W + g.w_off) + (n0 / 16) * 64 + lane;
+    v4f acc[RI][NSUB];
+#pragma unroll
+    for (int i = 0; i < RI; ++i)
+#pragma unroll
+        for (int j = 0; j < NSUB; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    const int chunks = g.K / 16;
+    GemmOperands<RI, NSUB> o0, o1;
+    gemm_load(o0, arow, B, 0, nblk);
+    int kc = 0;
+    for (; kc + 2 <= chunks; kc += 2) {
+        gemm_load(o1, arow, B, kc + 1, nblk);
+        gemm_chunk(acc, o0);
+        gemm_load(o0, arow, B, min(kc + 2, chunks - 1), nblk);
+        gemm_chunk(acc, o1);
+        // issue order: each load set, then the chunk that does not need it,
+        // so every load is one full chunk of MFMAs ahead of its use (left
+        // alone, the scheduler sinks the loads towards their use)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            __builtin_amdgcn_sched_group_barrier(0x020, RI + NSUB, 0);     // VMEM reads
+            __builtin_amdgcn_sched_group_barrier(0x008, 4 * RI * NSUB, 0);  // MFMA
+        }
+    }
+    if (kc < chunks) gemm_chunk(acc, o0);
+#pragma unroll
+    for (int i = 0; i < RI; ++i) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int q = 16 * i + 4 * kg + v;
+            if (q >= tile.count) continue;
+            const int pk = rows[tile.row_start + q];
+            float* orow = out + static_cast<std::size_t>(pk >> 4) * g.out_stride + g.out_base + (pk & 15) * g.out_mstride +
+                          n0 + r;
+#pragma unroll
+            for (int j = 0; j < NSUB; ++j) orow[16 * j] = acc[i][j][v];
+        }
+    }
+}
+
+// Shared-operand form for large linears: a workgroup of kGemmShareWaves waves
+// takes consecutive 16-row tiles of one group (a GemmTileSet) and one
+// 128-column block.  The B operands of each 16-wide K chunk (8 KB) are loaded
+// once per workgroup into LDS (double-buffered, one float4 per thread) and
+// read by every wave, so the weights cross L2 once per 128 rows instead of
+// once per 16.  The A rows, operand values and MFMA order per output tile are
+// those of k_node_gemm.  Waves past the set's tile count load and wait with
+// the others but store nothing.
+__global__ __launch_bounds__(64 * kGemmShareWaves) void k_node_gemm_shared(
+    const GemmTileSet* __restrict__ sets, const GemmTile* __restrict__ tiles, const GemmGroup* __restrict__ groups,
+    const int* __restrict__ rows, const float* __restrict__ W, const float* __restrict__ in, float* __restrict__ out) {
+    constexpr int NSUB = 8;
+    const GemmTileSet set = sets[blockIdx.x];
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const GemmTile tile = tiles[set.first + min(wave, set.count - 1)];
+    const GemmGroup g = groups[tile.group];
+    const int n0 = blockIdx.y * 16 * NSUB;
+    if (n0 >= g.N) return;  // uniform: the set's tiles share the group
+    const int r = lane & 15, kg = lane >> 4;
+    const float* arow;
+    {
+        const int q = min(r, tile.count - 1);
+        const int pk = rows[tile.row_start + q];
+        arow = in + static_cast<std::size_t>(pk >> 4) * g.in_stride + g.in_base + (pk & 15) * g.in_mstride + 4 * kg;
+    }
+    const int nblk = g.N / 16;
+    // chunk kc's operands of this column block: NSUB*64 float4, contiguous
+    const float4* B = reinterpret_cast<const float4*>(W + g.w_off) + (n0 / 16) * 64 + threadIdx.x;
+    __shared__ float4 sb[2][NSUB * 64];
+    static_assert(NSUB * 64 == 64 * kGemmShareWaves, "one B float4 per thread");
+    v4f acc[NSUB];
+#pragma unroll
+    for (int j = 0; j < NSUB; ++j) acc[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    const int chunks = g.K / 16;
+    // operands two chunks ahead: chunk kc runs from a0 and LDS buffer kc&1
+    // while the global loads of chunks kc+1 (a1, b1) and kc+2 (a2, b2) are
+    // in flight; b1 enters LDS at the end of chunk kc
+    const std::size_t bstep = static_cast<std::size_t>(nblk) * 64;
+    float4 a0 = *reinterpret_cast<const float4*>(arow);
+    float4 a1 = a0, b1 = B[0];
+    if (chunks > 1) {
+        a1 = *reinterpret_cast<const float4*>(arow + 16);
+        b1 = B[bstep];
+    }
+    sb[0][threadIdx.x] = B[0];
+    __syncthreads();
+    for (int kc = 0; kc < chunks; ++kc) {
+        float4 a2 = a1, b2 = b1;
+        if (kc + 2 < chunks) {
+            a2 = *reinterpret_cast<const float4*>(arow + 16 * (kc + 2));
+            b2 = B[static_cast<std::size_t>(kc + 2) * bstep];
+        }
+        float4 b[NSUB];
+#pragma unroll
+        for (int j = 0; j < NSUB; ++j) b[j] = sb[kc & 1][j * 64 + lane];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const float av = s == 0 ? a0.x : s == 1 ? a0.y : s == 2 ? a0.z : a0.w;
+#pragma unroll
+            for (int j = 0; j < NSUB; ++j) {
+                const float bv = s == 0 ? b[j].x : s == 1 ? b[j].y : s == 2 ? b[j].z : b[j].w;
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc[j], 0, 0, 0);
+            }
+        }
+        if (kc + 1 < chunks) sb[(kc + 1) & 1][threadIdx.x] = b1;
+        __syncthreads();
+        a0 = a1;
+        a1 = a2;
+        b1 = b2;
+    }
+    if (wave >= set.count) return;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int q = 4 * kg + v;
+        if (q >= tile.count) continue;
+        const int pk = rows[tile.row_start + q];
+        float* orow = out + static_cast<std::size_t>(pk >> 4) * g.out_stride + g.out_base + (pk & 15) * g.out_mstride +
+                      n0 + r;
+#pragma unroll
+        for (int j = 0; j < NSUB; ++j) orow[16 * j] = acc[j][v];
+    }
+}
+
+// Parts form, for models of kGemmPartsChannels channels and more: FP32 in and
+// out as products of bf16 parts (split_operand, v_mfma_f32_16x16x32_bf16 with
+// FP32 accumulators).  Six such MFMAs cover 32 input channels in 96 cycles
+// where the FP32 form needs 256, and 24 accumulator updates instead of 32 round
+// a sum of 128 terms.
 //
-// A workgroup of four waves takes a GemmTileSet, up to eight consecutive
-// 16-row tiles of one group (two a wave), and 16*NSUB columns.  The weights,
-// split and put in operand order when the model is loaded
+// A workgroup of four waves takes RT consecutive 16-row tiles a wave of one
+// GemmTileSet (the set with two, its halves with one) and 16*NSUB columns.
+// The weights, split and put in operand order when the model is loaded
 // (launch_pack_gemm_weights), cross LDS once per workgroup and 32-channel
 // chunk, the next chunk's weights and rows in flight while one runs; a wave
 // splits its own rows (44 VALU instructions a tile and chunk against 12*NSUB
 // MFMAs).  In a tile, lane l supplies channels 4*(l/16).. +3 and 16 + 4*(l/16).. +3 of
 // row or column l%16 (any order will do, the same for both; this one reads 64
 // contiguous bytes a row) and holds columns 4*(l/16).. +3 of row l%16.  Rows
-// past the set's count repeat its last row and store nothing.
-// ---------------------------------------------------------------------------
+// past the set's count repeat its last row and store nothing.  An output's
+// sum runs in the same order for every NSUB and RT, so a node's result does
+// not depend on how many rows the launch has.
+
 // acc[i] += (a[i] b)^T from the parts, the smallest products first.  The
 // weights are the MFMA's A operand, so a lane ends with four consecutive
 // columns of its row and stores them with 16 bytes.
@@ -1062,8 +1248,7 @@ __global__ __launch_bounds__(256) void k_pack_gemm_weights(std::size_t threads, 
     for (int p = 0; p < 3; ++p) out[(blk * 3 + p) * 64 + lane] = o.part[p];
 }
 
-constexpr int kGemmWaves = 4;
-constexpr int kGemmWaveTiles = kGemmSetTiles / kGemmWaves;  // 16-row tiles a wave
+constexpr int kGemmPartsWaves = 4;
 
 // address of a packed row (node << 4 | m) in the input or output of group g
 __device__ __forceinline__ std::size_t gemm_row(int pk, int stride, int base, int mstride) {
@@ -1086,25 +1271,29 @@ __device__ __forceinline__ void gemm_store(const v4f (&acc)[NSUB][RT], int i, co
     for (int j = 0; j < NSUB; ++j) *reinterpret_cast<v4f*>(orow + 16 * j) = acc[j][i];
 }
 
-template <int NSUB>
-__global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu(3)))
-void k_node_gemm(const GemmTileSet* __restrict__ sets, const GemmGroup* __restrict__ groups,
-                 const int* __restrict__ rows, const bf16x8* __restrict__ W, const float* __restrict__ in,
-                 float* __restrict__ out) {
-    constexpr int RT = kGemmWaveTiles, THREADS = 64 * kGemmWaves;
+template <int NSUB, int RT>
+__global__ __launch_bounds__(64 * kGemmPartsWaves) __attribute__((amdgpu_waves_per_eu(3)))
+void k_node_gemm_parts(const GemmTileSet* __restrict__ sets, const GemmGroup* __restrict__ groups,
+                       const int* __restrict__ rows, const bf16x8* __restrict__ W, const float* __restrict__ in,
+                       float* __restrict__ out) {
+    constexpr int THREADS = 64 * kGemmPartsWaves, ROWS = 16 * RT * kGemmPartsWaves;
+    constexpr int SPLIT = 16 * kGemmShareWaves / ROWS;  // workgroups of a set
     constexpr int BLK = NSUB * 3 * 64;                  // operand parts (16 bytes) of a chunk
-    constexpr int PER = (BLK + THREADS - 1) / THREADS;  // of them per thread
-    const GemmTileSet set = sets[blockIdx.x];
+    constexpr int PER = BLK / THREADS;                  // of them per thread
+    static_assert(SPLIT * ROWS == 16 * kGemmShareWaves && PER * THREADS == BLK);
+    const GemmTileSet set = sets[blockIdx.x / SPLIT];
+    const int first = ROWS * static_cast<int>(blockIdx.x % SPLIT), count = set.rows - first;
     const GemmGroup g = groups[set.group];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const int r = lane & 15, kg = lane >> 4;
     const int n0 = blockIdx.y * 16 * NSUB;
-    if (n0 >= g.N) return;  // uniform: the set's rows share the group
+    if (n0 >= g.N || count <= 0) return;  // uniform: the set's rows share the group
+    rows += set.row_start + first;
     const float* arow[RT];
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
         // rows past the set's count repeat its last row (their results are not stored)
-        const int pk = rows[set.row_start + min(16 * (RT * wave + i) + r, set.count - 1)];
+        const int pk = rows[min(16 * (RT * wave + i) + r, count - 1)];
         arow[i] = in + gemm_row(pk, g.in_stride, g.in_base, g.in_mstride) + 4 * kg;
     }
     const int nblk = g.N / 16, chunks = g.K / 32;
@@ -1120,14 +1309,14 @@ void k_node_gemm(const GemmTileSet* __restrict__ sets, const GemmGroup* __restri
 #pragma unroll
         for (int p = 0; p < PER; ++p) {
             const int q = static_cast<int>(threadIdx.x) + p * THREADS;
-            bn[p] = src[BLK % THREADS ? min(q, BLK - 1) : q];
+            bn[p] = src[q];
         }
     };
     auto commit = [&](int kc) __attribute__((always_inline)) {
 #pragma unroll
         for (int p = 0; p < PER; ++p) {
             const int q = static_cast<int>(threadIdx.x) + p * THREADS;
-            if (BLK % THREADS == 0 || q < BLK) sb[kc & 1][q] = bn[p];
+            sb[kc & 1][q] = bn[p];
         }
     };
     v4f acc[NSUB][RT];
@@ -1168,96 +1357,8 @@ void k_node_gemm(const GemmTileSet* __restrict__ sets, const GemmGroup* __restri
     }
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
-        const int first = 16 * (RT * wave + i);
-        gemm_store<NSUB, RT>(acc, i, rows + set.row_start + first, set.count - first, g, out + n0, r, kg);
-    }
-}
-
-// The form for few rows, where the chip is not full and the latency of one
-// tile is the time: FP32 MFMAs (v_mfma_f32_16x16x4_f32), a wave per 16-row
-// tile and 16*NSUB columns, nothing shared.  Step s of a 16-channel chunk uses
-// channel 4*(l/16) + s, so a lane reads four consecutive inputs of its row with
-// 16 bytes, and the weights lie so (swizzle_gemm_weights) that a chunk and
-// 16-column block is one contiguous 1 KB load a wave; a lane holds rows
-// 4*(l/16).. +3 of column l%16.  Two operand sets alternate: the loads of chunk
-// kc+1 are in flight while chunk kc runs.  (The parts' form with one tile a
-// wave and its operands straight from L2 took 42 us instead of 44 for the six
-// linears of 320 medium-model nodes, but the R1 reverse pass behind it 122
-// instead of 114: not kept.)
-template <int NSUB>
-struct GemmOperands {
-    float4 a, b[NSUB];
-};
-
-template <int NSUB>
-__device__ __forceinline__ void gemm_load(GemmOperands<NSUB>& o, const float* arow, const float4* __restrict__ B, int kc,
-                                          int nblk) {
-    o.a = *reinterpret_cast<const float4*>(arow + 16 * kc);
-#pragma unroll
-    for (int j = 0; j < NSUB; ++j) o.b[j] = B[(static_cast<std::size_t>(kc) * nblk + j) * 64];
-}
-
-template <int NSUB>
-__device__ __forceinline__ void gemm_chunk(v4f (&acc)[NSUB], const GemmOperands<NSUB>& o) {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const float av = s == 0 ? o.a.x : s == 1 ? o.a.y : s == 2 ? o.a.z : o.a.w;
-#pragma unroll
-        for (int j = 0; j < NSUB; ++j) {
-            const float bv = s == 0 ? o.b[j].x : s == 1 ? o.b[j].y : s == 2 ? o.b[j].z : o.b[j].w;
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc[j], 0, 0, 0);
-        }
-    }
-}
-
-template <int NSUB>
-__global__ __launch_bounds__(64) void k_node_gemm_wave(const GemmTileSet* __restrict__ sets,
-                                                       const GemmGroup* __restrict__ groups,
-                                                       const int* __restrict__ rows, const float* __restrict__ W,
-                                                       const float* __restrict__ in, float* __restrict__ out) {
-    // blockIdx.x: row tile; blockIdx.y: 16*NSUB-column block.  (Dispatch
-    // order x-fastest: concurrent waves share one column block's weights.
-    // Grouping a tile's column blocks on one XCD measured slower.)
-    const GemmTileSet set = sets[blockIdx.x / kGemmSetTiles];
-    const int first = 16 * static_cast<int>(blockIdx.x % kGemmSetTiles);
-    if (first >= set.count) return;
-    const int count = min(16, set.count - first);
-    rows += set.row_start + first;
-    const GemmGroup g = groups[set.group];
-    const int n0 = blockIdx.y * 16 * NSUB;
-    if (n0 >= g.N) return;
-    const int lane = threadIdx.x, r = lane & 15, kg = lane >> 4;
-    // rows past the tile's count repeat its last row (their results are not stored)
-    const float* arow = in + gemm_row(rows[min(r, count - 1)], g.in_stride, g.in_base, g.in_mstride) + 4 * kg;
-    const int nblk = g.N / 16;
-    const float4* B = reinterpret_cast<const float4*>(W + g.w_off) + (n0 / 16) * 64 + lane;
-    v4f acc[NSUB];
-#pragma unroll
-    for (int j = 0; j < NSUB; ++j) acc[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    const int chunks = g.K / 16;  // even: K is a multiple of 32
-    GemmOperands<NSUB> o0, o1;
-    gemm_load(o0, arow, B, 0, nblk);
-    for (int kc = 0; kc < chunks; kc += 2) {
-        gemm_load(o1, arow, B, kc + 1, nblk);
-        gemm_chunk(acc, o0);
-        gemm_load(o0, arow, B, min(kc + 2, chunks - 1), nblk);
-        gemm_chunk(acc, o1);
-        // issue order: each load set, then the chunk that does not need it,
-        // so every load is one full chunk of MFMAs ahead of its use (left
-        // alone, the scheduler sinks the loads towards their use)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            __builtin_amdgcn_sched_group_barrier(0x020, 1 + NSUB, 0);  // VMEM reads
-            __builtin_amdgcn_sched_group_barrier(0x008, 4 * NSUB, 0);  // MFMA
-        }
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int q = 4 * kg + v;
-        if (q >= count) continue;
-        float* orow = out + gemm_row(rows[q], g.out_stride, g.out_base, g.out_mstride) + n0 + r;
-#pragma unroll
-        for (int j = 0; j < NSUB; ++j) orow[16 * j] = acc[j][v];
+        const int t = 16 * (RT * wave + i);
+        gemm_store<NSUB, RT>(acc, i, rows + t, count - t, g, out + n0, r, kg);
     }
 }
 
@@ -1913,43 +2014,88 @@ bool kernel_paths(int l_max, int L_max, std::vector<int>& le, std::vector<int>& 
     return false;
 }
 
+// The form a linear runs in.  Up to 128 channels FP32 MFMAs: in calls back to
+// back the bf16 ones of the parts' form cost more than they gain.  The core
+// clock of every kernel of the call falls, measured inside them from 2,320 to
+// 2,080 MHz in R1 reverse and from 2,150 to 1,910 in R0 forward, and stays
+// there; with 4 ms of idle time between calls both forms run at 2,070 and
+// 1,920.  5,000 atoms of the 128-channel, l_max 3 shape: six linears 272 us in
+// FP32 and 185 in parts, R1 reverse 624 and 676, R0 reverse 198 and 213, the
+// call 1,880 and 1,904; 6,791 atoms 2,608 and 2,677, field response of 1,080
+// atoms 4,314 and 4,480, 13,720 atoms 4,763 and 4,830 (29,160 atoms 10,115 and
+// 9,947: the larger linears win there, but a node's result would depend on
+// the launch's rows).  How far the clock falls differs from card to card.  A
+// linear's work goes with the square of the channels, the edge kernels' with
+// their number: at 256 channels the call gains all the same, 1,050 atoms
+// 1,640 us in FP32 and 1,585 in parts, 1,500 atoms 1,914 and 1,858, 6,000 atoms
+// 6,967 and 6,621, 30,000 atoms 33,865 and 32,305 (360 atoms 782 and 779, 120
+// atoms 650 and 670).
+NodeGemmForm node_gemm_form(const GemmPlan& plan, bool parts) {
+    const long long blocks128 = (plan.max_n + 127) / 128;
+    if (parts) {
+        // Workgroups of 128 rows and 128 columns while that gives every CU two
+        // of them, of 64 rows down to one, then of 64 x 64 (600 atoms of 256
+        // channels: 1,034 us a call; 1,055 without the smallest, 1,063 with
+        // 128 x 64 for all below two a CU; 120 atoms 670, 698 and 708).
+        const long long full = plan.num_sets * blocks128;
+        if (full >= 512) return {2, 8, 8};
+        if (full >= 256) return {2, 8, 4};
+        return {2, 4, 4};
+    }
+    const long long waves128 = plan.num_tiles * blocks128;
+    // Large linears (at least ~32 waves per SIMD): the shared-operand kernel
+    // (50,000 atoms of 128 channels: 17,013 us a call, 17,977 without it;
+    // slower at 80,000 rows).
+    if (plan.n_sub == 8 && waves128 >= 32 * 1024) return {1, 8, kGemmShareWaves};
+    // Narrower waves (64 columns) when 128-column waves would give fewer than
+    // about 8 per SIMD (1024 SIMDs): more waves fill the chip better than the
+    // wider tile's operand reuse pays (the 5,000-node linears run 8% faster).
+    if (plan.n_sub == 8 && (plan.narrow || waves128 < 8 * 1024)) return {0, 4, 1};
+    return {0, plan.n_sub, 1};
+}
+
 void launch_node_gemm(const GemmPlan& plan, const GemmWeights& W, const float* in, float* out, hipStream_t s) {
-    if (plan.num_sets == 0) return;
-    auto blocks = [&](int n_sub) { return (plan.max_n + 16 * n_sub - 1) / (16 * n_sub); };
-    auto wave = [&](auto n) {
-        constexpr int NSUB = n;
-        k_node_gemm_wave<NSUB><<<dim3(plan.num_sets * kGemmSetTiles, blocks(NSUB)), 64, 0, s>>>(
-            plan.sets, plan.groups, plan.rows, W.fp32, in, out);
+    if (plan.num_tiles == 0) return;
+    const NodeGemmForm form = node_gemm_form(plan, W.parts != nullptr);
+    const unsigned blocks = (plan.max_n + 16 * form.n_sub - 1) / (16 * form.n_sub);
+    auto parts = [&](auto n, auto rt) {
+        constexpr int NSUB = n, RT = rt, SPLIT = kGemmShareWaves / (RT * kGemmPartsWaves);
+        k_node_gemm_parts<NSUB, RT><<<dim3(plan.num_sets * SPLIT, blocks), 64 * kGemmPartsWaves, 0, s>>>(
+            plan.sets, plan.groups, plan.rows, static_cast<const bf16x8*>(W.parts), in, out);
     };
-    auto shared = [&](auto n) {
+    auto waves = [&](auto n) {
         constexpr int NSUB = n;
-        k_node_gemm<NSUB><<<dim3(plan.num_sets, blocks(NSUB)), 64 * kGemmWaves, 0, s>>>(
-            plan.sets, plan.groups, plan.rows, static_cast<const bf16x8*>(W.packed), in, out);
+        k_node_gemm<NSUB><<<dim3(plan.num_tiles, blocks), 64, 0, s>>>(plan.tiles, plan.groups, plan.rows, W.fp32, in,
+                                                                      out);
     };
-    // Few rows: the wave form until 64-column workgroups would give every CU
-    // two (the six linears of 320 medium-model nodes 44 us in it; a workgroup
-    // form's launch takes about 10 us at any number of rows below, a wave
-    // form's 5 to 10).  Above, 128 columns a workgroup once that gives each CU two of them,
-    // else 64 (128 x 128 with the launch's 5.9 us: 20,000 rows 14.0 against
-    // 13.6 us, 80,000 rows 26 against 28.6).
-    const int n4 = plan.n_sub >= 4 ? 4 : 2;
-    const bool few = static_cast<long long>(plan.num_sets) * blocks(n4) < kGemmWaveFill;
-    if (few && n4 == 4)
-        wave(std::integral_constant<int, 4>{});
-    else if (few)
-        wave(std::integral_constant<int, 2>{});
-    else if (plan.n_sub >= 8 && static_cast<long long>(plan.num_sets) * blocks(8) >= kGemmFill)
-        shared(std::integral_constant<int, 8>{});
-    else if (n4 == 4)
-        shared(std::integral_constant<int, 4>{});
+    if (form.kind == 2) {
+        if (form.tiles == 8)
+            parts(std::integral_constant<int, 8>{}, std::integral_constant<int, 2>{});
+        else if (form.n_sub == 8)
+            parts(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
+        else
+            parts(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
+        SMX_LAUNCH_CHECK("node_gemm_parts");
+        return;
+    }
+    if (form.kind == 1) {
+        k_node_gemm_shared<<<dim3(plan.num_sets, blocks), 64 * kGemmShareWaves, 0, s>>>(
+            plan.sets, plan.tiles, plan.groups, plan.rows, W.fp32, in, out);
+        SMX_LAUNCH_CHECK("node_gemm_shared");
+        return;
+    }
+    if (form.n_sub == 8)
+        waves(std::integral_constant<int, 8>{});
+    else if (form.n_sub == 4)
+        waves(std::integral_constant<int, 4>{});
     else
-        shared(std::integral_constant<int, 2>{});
+        waves(std::integral_constant<int, 2>{});
     SMX_LAUNCH_CHECK("node_gemm");
 }
 
 void launch_pack_gemm_weights(const float* w, std::size_t count, int K, int N, void* out, hipStream_t s) {
-    if (K % 32 != 0 || N % 32 != 0)
-        throw std::invalid_argument("node linears take multiples of 32 inputs and outputs");
+    if (K % 32 != 0 || N % 128 != 0)
+        throw std::invalid_argument("node linears of bf16 parts take multiples of 32 inputs and of 128 outputs");
     const std::size_t threads = count * (K / 32) * (N / 16) * 64;
     if (threads == 0) return;
     k_pack_gemm_weights<<<blocks_for(static_cast<std::int64_t>(threads), 256), 256, 0, s>>>(
@@ -1958,6 +2104,7 @@ void launch_pack_gemm_weights(const float* w, std::size_t count, int K, int N, v
 }
 
 void swizzle_gemm_weights(const float* w, int K, int N, float* out) {
+    if (K % 16 != 0 || N % 16 != 0) throw std::invalid_argument("node-linear dimensions must be multiples of 16");
     const int nblk = N / 16;
     for (int kc = 0; kc < K / 16; ++kc)
         for (int nb = 0; nb < nblk; ++nb)

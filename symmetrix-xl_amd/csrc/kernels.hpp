@@ -19,12 +19,12 @@ struct FieldEntryDev {
     float coef;
 };
 
-// Weight blocks of the node linears in the operand order of the two GEMM
-// kernels: three bf16 parts per weight (6 bytes, launch_pack_gemm_weights) for
-// the workgroup form, FP32 (swizzle_gemm_weights) for the one-wave form.
+// Weight blocks of the node linears in the operand order of the form that the
+// model takes: FP32 (swizzle_gemm_weights), or three bf16 parts per weight (6
+// bytes, launch_pack_gemm_weights) from kGemmPartsChannels channels on.
 struct GemmWeights {
-    const void* packed = nullptr;
     const float* fp32 = nullptr;
+    const void* parts = nullptr;
 };
 
 // Model tables resident in HBM (owned by the evaluator).
@@ -47,12 +47,12 @@ struct DeviceModel {
     GemmWeights H1_w;
     GemmWeights H1_wt;
     // pre_linear_up basis: x = M0[:,0,:] P0 and M0_adj[:,0,:] += P0 d (GEMM
-    // weights P0 and P0^T, packed); residual: per-type H1 and x offsets
+    // weights P0 and P0^T, in operand order); residual: per-type H1 and x offsets
     bool pre_linear_up = false, residual = false;
     // one interaction: M1 of H1, no R1 / A1 (single_layer_readout)
     bool single_layer = false;
     // MACEField: H1p = M0 P (+ b), H1f = H1p + field terms, x = H1f[:,0,:],
-    // H1 = H1f U (GEMM weights packed: P, U per l; W per path)
+    // H1 = H1f U (GEMM weights in operand order: P, U per l; W per path)
     bool field = false;
     GemmWeights P_w;
     GemmWeights P_wt;
@@ -126,30 +126,42 @@ struct DeviceGraph {
 // Node linears: out[row, n] = sum_k in[row, k] W[k, n] over the rows of one
 // weight group.  A row is (tile-local node, m) packed as node << 4 | m; its
 // input starts at node*in_stride + in_base + m*in_mstride (likewise the
-// output).  W is packed by launch_pack_gemm_weights.
+// output).  W is stored in MFMA operand order (GemmWeights).
 struct GemmGroup {
     std::int64_t w_off;  // element offset of the group's [K][N] block
     int K, N;
     int in_stride, in_base, in_mstride;
     int out_stride, out_base, out_mstride;
 };
-// Up to kGemmSetTiles 16-row tiles of one group: a workgroup of the GEMM
-// kernel, rows [row_start, row_start+count) of the plan's row list.
-constexpr int kGemmSetTiles = 8;
-constexpr int kGemmSetRows = 16 * kGemmSetTiles;
-// workgroups from which a launch takes the workgroup form (two per CU), and
-// from which their column blocks widen (two per CU)
-constexpr long long kGemmWaveFill = 512, kGemmFill = 512;
-struct GemmTileSet {
-    int row_start, count, group;
+// rows per wave tile (a multiple of 16): 16 rows x up to 128 columns per
+// wave.  At the medium shape this reads each input row once per 128 output
+// columns and still gives about five waves per SIMD; it measured faster than
+// 32 x 64 and 64 x 64 tiles.
+constexpr int kGemmRows = 16;
+struct GemmTile {
+    int row_start, count, group;  // rows [row_start, row_start+count), count <= kGemmRows
 };
+// Up to kGemmShareWaves consecutive tiles of one group: the workgroup of the
+// shared-operand and the parts' GEMM kernel (tile indices relative to
+// GemmPlan::tiles; rows [row_start, row_start+rows) of the plan's row list).
+constexpr int kGemmShareWaves = 8;
+struct GemmTileSet {
+    int first, count;
+    int row_start, rows, group;
+};
+// Channels from which a model's node linears run as products of bf16 parts
+// (the reason stands at launch_node_gemm).
+constexpr int kGemmPartsChannels = 256;
 struct GemmPlan {
+    const GemmTile* tiles = nullptr;
     const GemmGroup* groups = nullptr;
     const int* rows = nullptr;        // packed (node << 4 | m)
+    int num_tiles = 0;
     int max_n = 0;
-    int n_sub = 2;  // most 16-column tiles per wave (8, 4 or 2): divides every group's N/16
-    const GemmTileSet* sets = nullptr;  // the workgroups' tiles
+    int n_sub = 2;  // 16-column tiles per wave (8, 4 or 2): divides every group's N/16
+    const GemmTileSet* sets = nullptr;  // tiles grouped for the workgroup kernels
     int num_sets = 0;
+    bool narrow = false;  // prefer 64-column waves to 128-column ones (long K)
 };
 
 // Readout batches: up to kReadoutBatch receivers of one type, as a range of
@@ -338,11 +350,11 @@ void set_last_error(const std::string& message);
 std::unique_ptr<KernelSet> make_kernel_set(int C, int l_max, int L_max, const std::vector<std::int32_t>& m0_terms,
                                            const std::vector<std::int32_t>& m0_offsets,
                                            const std::vector<std::int32_t>& m1_terms);
-// count row-major [K][N] blocks (device) -> the GEMM's operand order
+// count row-major [K][N] blocks (device) -> the parts' operand order
 // [K/32][N/16][3 parts][64 lanes][8] bf16 of each (device, 6 bytes a weight)
 void launch_pack_gemm_weights(const float* w, std::size_t count, int K, int N, void* out, hipStream_t s);
-// one row-major [K][N] block -> FP32 order [K/16][N/16][4][16][4] of the
-// one-wave form (k chunk, column block, lane/16, lane%16, k within the lane's four)
+// [K][N] row-major block -> FP32 MFMA B-operand order [K/16][N/16][4][16][4]
+// (k chunk, column block, lane/16, lane%16, k within the lane's four)
 void swizzle_gemm_weights(const float* w, int K, int N, float* out);
 // paths of the compiled kernel set for (l_max, L_max), false if none
 bool kernel_paths(int l_max, int L_max, std::vector<int>& le, std::vector<int>& ls, std::vector<int>& lo);
@@ -365,6 +377,13 @@ void geometry_records(int l_max, std::int64_t E, const double* xyz, const double
 void launch_edge_pairs(std::int64_t E, const int* receivers, const int* node_types, const int* neigh_types,
                        const int* type_to_active, int active_types, int* edge_pair, int* bad, hipStream_t s);
 
+// how launch_node_gemm runs a plan: FP32 waves (kind 0), the FP32
+// shared-operand workgroup (1) or the parts' (2), with n_sub 16-column and
+// `tiles` 16-row tiles of the plan a workgroup
+struct NodeGemmForm {
+    int kind, n_sub, tiles;
+};
+NodeGemmForm node_gemm_form(const GemmPlan& plan, bool parts);
 void launch_node_gemm(const GemmPlan& plan, const GemmWeights& W, const float* in, float* out, hipStream_t s);
 // rows[li][0..row_len) += bias[types[r0 + li]][0..row_len) for li < nr
 void launch_type_bias(int r0, int nr, const int* types, int row_len, const float* bias, float* rows, hipStream_t s);

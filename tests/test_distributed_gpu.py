@@ -421,6 +421,33 @@ def test_medium_slabs_sum_to_the_whole_system(medium_model_path):
     np.testing.assert_allclose(st, sw, rtol=0, atol=1e-8)
 
 
+@pytest.mark.parametrize("model,parts", [("medium", 2), ("medium", 3), ("wide", 2), ("wide", 3)])
+def test_a_nodes_energy_does_not_depend_on_the_split(request, model, parts):
+    """Node energies of 5,000 atoms (128 channels) and 1,050 atoms (256
+    channels) bit for bit those of the slabs: the sums behind a node run in
+    one order whatever the number of rows that a linear has (78,000 down to
+    1,050 here, on both sides of the lines between its launch forms)."""
+    from symmetrix import systems
+    from symmetrix.mace_kokkos import MACEKokkosFloat, neighbor_list
+    path = request.getfixturevalue(model + "_model_path")
+    s = _system("medium") if model == "medium" else systems.water_box(num_molecules=350, seed=3)
+    whole = MACEKokkosFloat(path)
+    lut = {int(z): i for i, z in enumerate(whole.atomic_numbers)}
+    types = np.array([lut[int(z)] for z in s["numbers"]], np.int32)
+    cell = np.asarray(s["cell"], float)
+    g = neighbor_list(np.asarray(s["positions"], float), cell, whole.r_cut)
+    xyz = g["fractional_xyz"] @ cell
+    ref = {"graph": g, "xyz": xyz.ravel(), "r": np.linalg.norm(xyz, axis=1)}
+    n = len(types)
+    gen = whole._prepare_factorized_graph(n, types, g["num_neigh"], g["sources"], types[g["sources"]])
+    whole._compute_prepared_factorized(gen, ref["xyz"], ref["r"])
+    ew, fw = whole.node_energies, whole._reduce_atom_forces(n, None, None, gen)
+    whole.close()
+    e, f, _ = _run(path, s, ref, types, parts)
+    np.testing.assert_array_equal(e, ew)
+    np.testing.assert_allclose(f, fw, rtol=0, atol=1e-6)
+
+
 @pytest.mark.parametrize("model", ["tiny", "tiny_residual"])
 def test_pair_style_modes_give_the_same_virial(request, model):
     """One rank, the same LAMMPS arrays: the virial the pair style's
