@@ -89,9 +89,17 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 
 // FP32 matrix products on bf16 MFMAs: an FP32 value as three bf16 parts, each
-// the rounding of what the ones before it left.
+// the rounding of what the ones before it left.  Three parts hold a normal
+// value exactly while the last one's bits stay above 2^-133 (values from about
+// 2^-110 on; smaller ones keep that absolute precision).  The first two are
+// kept finite, so that values up to FLT_MAX, which round to infinity in bf16,
+// stay finite too, and an infinity or NaN is the third part alone: it meets
+// only the other operand's first part and gives what an FP32 product gives.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
+
+// largest bf16, and the largest that a second part can be
+constexpr float kSplitMax = 0x1.fep127f, kSplitMax2 = 0x1p120f;
 
 struct SplitOperand {
     bf16x8 part[3];
@@ -109,7 +117,10 @@ __device__ __forceinline__ SplitOperand split_operand(f32x8 x) {
         u32x4 bits;
 #pragma unroll
         for (int h = 0; h < 4; ++h) {
-            const f32x2 v = {x[2 * h], x[2 * h + 1]};
+            const float big = p == 0 ? kSplitMax : kSplitMax2;
+            const f32x2 v = p == 2 ? f32x2{x[2 * h], x[2 * h + 1]}
+                                   : f32x2{__builtin_amdgcn_fmed3f(x[2 * h], -big, big),
+                                           __builtin_amdgcn_fmed3f(x[2 * h + 1], -big, big)};
             bits[h] = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
             if (p < 2) {
                 x[2 * h] -= __uint_as_float(bits[h] << 16);
@@ -122,7 +133,9 @@ __device__ __forceinline__ SplitOperand split_operand(f32x8 x) {
 }
 
 // acc + a b over 32 channels (v_mfma_f32_16x16x32_bf16) from the parts, the
-// smallest products first; the products left out are below 2^-26 |a b|.
+// smallest products first.  A second part is at most 2^-8 and a third 2^-17 of
+// its value: the products left out (2 with 3, 3 with 2, 3 with 3) are at most
+// about 2^-24 |a b|, the size of an FP32 product's own rounding.
 typedef float acc4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ acc4 split_product(const SplitOperand& a, const SplitOperand& b, acc4 acc) {
     constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};

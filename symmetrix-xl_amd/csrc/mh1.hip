@@ -1852,8 +1852,10 @@ int pack_parts(const float* W, int M, int K, std::vector<std::uint16_t>& out) {
                     if (row >= M || k >= K) continue;
                     float x = W[static_cast<std::size_t>(row) * K + k];
                     for (int p = 0; p < 3; ++p) {
+                        const float big = p == 0 ? kSplitMax : p == 1 ? kSplitMax2 : INFINITY;
+                        const float v = x > big ? big : x < -big ? -big : x;
                         std::uint32_t u;
-                        std::memcpy(&u, &x, 4);
+                        std::memcpy(&u, &v, 4);
                         u = (u + 0x7fffu + (u >> 16 & 1u)) & 0xffff0000u;  // nearest, ties to even
                         float part;
                         std::memcpy(&part, &u, 4);

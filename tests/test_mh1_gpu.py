@@ -10,6 +10,8 @@ cutoff on the weights with Agnesi distances, a linear bias and ZBL, and the
 density, layer features, edge weights) localise a failure.
 """
 
+import json
+
 import numpy as np
 import pytest
 
@@ -351,3 +353,30 @@ def test_mh1_edge_mlp_at_tile_edges(paths, name, n):
         got = ev._stage("w%d" % k).reshape(ref.shape)
         assert np.abs(got - ref).max() <= 4 * 64 * 2.0 ** -24 * max(1.0, np.abs(ref).max())
     assert np.abs(f - f_ref).max() < 1e-4 * max(1.0, np.abs(f_ref).max())
+
+
+@pytest.mark.parametrize("name", ["mh1_tiny_mlp32", "mh1_medium"])
+def test_mh1_edge_mlp_weight_beyond_bf16(paths, name, tmp_path):
+    """A final-linear weight of 3.4e38, which rounds to infinity in bf16, gives
+    what FP32 products give."""
+    with open(paths[name]) as f:
+        d = json.load(f)
+    last = d["interactions"][0]["conv_tp_weights"]["layers"][-1]["weight"]
+    cols, hidden = int(last["shape"][0]), int(last["shape"][1])
+    last["values"][3 * hidden + 1] = 3.4e38
+    path = str(tmp_path / "huge.json")
+    with open(path, "w") as f:
+        json.dump(d, f)
+    model = mo.MH1Oracle(path)
+    pos, cell, types = _random_system(model, 7, 8.0, 5)
+    g, xyz, r = _graph(model, pos, cell)
+    with np.errstate(all="ignore"):
+        model.evaluate(types, g["receivers"], g["sources"], xyz)
+    ev, _, _ = _gpu(path, types, g, xyz, r)
+    ref = np.asarray(model.stages["states"][0]["wraw"]).reshape(-1, cols)
+    got = ev._stage("w0").reshape(-1, cols)
+    fits = np.abs(ref[:, 3]) < 3e38
+    assert fits.sum() > len(r) // 2 and np.abs(ref[fits, 3]).max() > 1e37
+    np.testing.assert_allclose(got[fits, 3], ref[fits, 3], rtol=4e-5)
+    rest = np.arange(cols) != 3
+    np.testing.assert_allclose(got[:, rest], ref[:, rest], rtol=0, atol=4 * 64 * 2.0 ** -24 * np.abs(ref[:, rest]).max())
