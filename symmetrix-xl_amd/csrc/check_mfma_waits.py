@@ -1,17 +1,18 @@
 #!/usr/bin/env python3
-"""Checks this library's gfx950 assembly for MFMA results read too early.
+"""Checks this library's gfx950 assembly for MFMA results touched too early.
 
-An instruction that reads a register written by v_mfma_f32_16x16x4_f32 (8
-passes) must issue at least ten wait states after it, on every path, and one
-that touches a register written by v_mfma_f32_16x16x32_bf16 (4 passes) at least
-eight; the hardware does not interlock.  The compiler inserts the waits, but in kernels
+An instruction other than an MFMA that reads or overwrites a register written
+by v_mfma_f32_16x16x4_f32 (8 passes) must issue at least ten wait states after
+it, on every path, and after v_mfma_f32_16x16x32_bf16 (4 passes) at least eight;
+the hardware does not interlock.  The compiler inserts the waits, but in kernels
 whose MFMA chains sat in runtime-conditional blocks it padded only the
 fall-through path into a join, and a read on the taken branch came one
 instruction after its MFMA (a stale accumulator element, silently wrong).
 This walks each kernel's control-flow graph backwards from every instruction
-that reads a register (VALU sources, memory addresses and data) and reports
-the reads with fewer than MIN wait states since an MFMA that writes the
-register, over any path; an s_nop N counts N + 1, other instructions one.
+that touches a register (VALU operands, memory addresses and data) and reports
+those with fewer than MIN wait states since an MFMA that writes the register,
+over any path (a bf16 MFMA counts two more); an s_nop N counts N + 1, other
+instructions one.
 
     python3 check_mfma_waits.py file.s [--min 10]      (exit 1 on findings)
 
@@ -94,7 +95,7 @@ def _blocks(body):
 
 
 def findings(body, minimum):
-    """(block label, instruction, register, wait states) for each early read."""
+    """(block label, instruction, register, wait states) for each early read or overwrite."""
     blocks, preds = _blocks(body)
 
     def since_mfma(bi, idx, reg, budget, seen):
@@ -119,7 +120,7 @@ def findings(body, minimum):
             if t.startswith("v_mfma") or t.startswith("s_") or " " not in t:
                 continue
             ops = t.split(None, 1)[1].split(",")
-            for op in (ops[1:] if t.startswith("v_") else ops):
+            for op in ops:
                 for reg in _regs(op):
                     d = since_mfma(bi, k, reg, minimum, frozenset())
                     if d < minimum:  # (a bf16 MFMA's distance counts its slack)
@@ -139,7 +140,7 @@ def main(argv=None):
         for name, body in kernels:
             for label, ins, reg, d in findings(body, args.min):
                 bad += 1
-                print("%s: %s: %s: %s read %d wait states after its MFMA" % (path, name, label, ins, d))
+                print("%s: %s: %s: %s touched %d wait states after its MFMA" % (path, name, label, ins, d))
         print("%s: %d functions checked" % (path, len(kernels)))
     return 1 if bad else 0
 

@@ -90,8 +90,8 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // FP32 matrix products on bf16 MFMAs: an FP32 value as three bf16 parts, each
 // the rounding of what the ones before it left.  Three parts hold a normal
-// value exactly while the last one's bits stay above 2^-133 (values from about
-// 2^-110 on; smaller ones keep that absolute precision).  The first two are
+// value exactly; the MFMA takes parts below 2^-126 as zero, so values below
+// about 2^-102 lose their last bits (2^-16 of a sum at inputs of 2^-112).  The first two are
 // kept finite, so that values up to FLT_MAX, which round to infinity in bf16,
 // stay finite too, and an infinity or NaN is the third part alone: it meets
 // only the other operand's first part and gives what an FP32 product gives.

@@ -1,5 +1,6 @@
-"""Reads of MFMA results in this library's gfx950 assembly wait ten states on
-every path (symmetrix-xl_amd/csrc/check_mfma_waits.py).
+"""Reads and overwrites of MFMA results in this library's gfx950 assembly wait
+on every path: ten states after an FP32 MFMA, eight after a bf16 one
+(symmetrix-xl_amd/csrc/check_mfma_waits.py).
 
 A read that comes too early returns a stale accumulator element with no
 error.  The compiler has padded only the fall-through path into a join: the
@@ -59,6 +60,45 @@ STORE_ON_BRANCH = """_Zk:
 """
 
 
+# a bf16 MFMA's result read at seven wait states, and at eight
+BF16_SEVEN = """_Zk:
+\tv_mfma_f32_16x16x32_bf16 v[8:11], v[0:3], v[4:7], 0
+\ts_nop 6
+\tv_add_f32_e32 v3, v9, v3
+\ts_endpgm
+"""
+BF16_EIGHT = BF16_SEVEN.replace("s_nop 6", "s_nop 7")
+
+# the taken branch skips the padding; an FP32 MFMA on the other path asks for ten
+BF16_TAKEN_BRANCH = """_Zk:
+\tv_mfma_f32_16x16x32_bf16 a[0:3], v[0:3], v[4:7], a[0:3]
+\ts_cbranch_vccnz .LBB0_2
+\ts_nop 7
+.LBB0_2:
+\tv_accvgpr_read_b32 v4, a2
+\ts_endpgm
+"""
+MIXED = """_Zk:
+\ts_cbranch_vccnz .LBB0_1
+\tv_mfma_f32_16x16x32_bf16 v[8:11], v[0:3], v[4:7], 0
+\ts_branch .LBB0_2
+.LBB0_1:
+\tv_mfma_f32_16x16x4_f32 v[12:15], v1, v2, 0
+.LBB0_2:
+\ts_nop 6
+\tv_add_f32_e32 v3, v9, v13
+\ts_endpgm
+"""
+
+# an accumulator overwritten, not read, right after its MFMA
+OVERWRITE = """_Zk:
+\tv_mfma_f32_16x16x4_f32 v[8:11], v1, v2, 0
+\ts_nop 4
+\tv_mov_b32_e32 v10, 0
+\ts_endpgm
+"""
+
+
 def _check(text):
     (name, body), = cw.split_kernels(text.split("\n"))
     return cw.findings(body, 10)
@@ -74,6 +114,21 @@ def test_planted_early_reads_are_found():
 
 def test_settled_chains_pass():
     assert _check(SETTLED) == []
+
+
+def test_bf16_mfmas_ask_for_eight_states():
+    # (reported with the two that a bf16 MFMA asks less)
+    assert [(reg, d) for _, _, reg, d in _check(BF16_SEVEN)] == [("v9", 9)]
+    assert _check(BF16_EIGHT) == []
+    assert [(ins.split()[0], reg, d) for _, ins, reg, d in _check(BF16_TAKEN_BRANCH)] == [
+        ("v_accvgpr_read_b32", "a2", 3)]
+    # seven states after the join: eight (with the branch) after the bf16 MFMA, seven after the FP32 one
+    assert [(reg, d) for _, _, reg, d in _check(MIXED)] == [("v13", 7)]
+
+
+def test_overwrites_are_found():
+    assert [(ins.split()[0], reg, d) for _, ins, reg, d in _check(OVERWRITE)] == [("v_mov_b32_e32", "v10", 5)]
+    assert _check(OVERWRITE.replace("s_nop 4", "s_nop 9")) == []
 
 
 @pytest.mark.skipif(shutil.which("make") is None or not os.path.exists("/opt/rocm/bin/hipcc"),
