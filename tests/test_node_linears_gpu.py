@@ -1,13 +1,13 @@
-"""Node linears on the GPU against float64 products of the kernel's own inputs.
+"""Node linears on the GPU against float64 products of the kernels' own inputs.
 
-H1 = M0 H1_w per degree (the linear whose rows are every node's): row counts
-at the edges of its 16-row tiles and 128-row sets, and sizes that take each
-form of the kernel (FP32 waves of 32 and 64 columns, workgroups of 32, 64 and
-128 columns on bf16 parts).
+A0 = Phi0 W per (type, l), H1 = M0 W and A1 = Phi1 W per l, and the reverse of
+A1 (dPhi1 = A1_adj W^T): row counts at the edges of 16-row tiles and of the
+workgroups' 64 and 128 rows, and sizes that take each form of the kernel, which
+a case names: FP32 waves of 32, 64 and 128 columns, the FP32 workgroup, and at
+256 channels the workgroups on bf16 parts.
 
-Bound: a sum over K inputs rounds an FP32 accumulator K times (FP32 products)
-or 6 K / 32 times (products of parts, which drop less than 2^-25 |x w| too),
-each time by at most 2^-24 of a partial sum, itself at most sum |x w|.
+Bound (test_bf16_parts.ROUNDING, which tells a lost product of parts): the root
+mean square of the error is at most 1.5 * 2^-24 of that of sum |x w|.
 """
 
 import functools
@@ -16,43 +16,99 @@ import json
 import numpy as np
 import pytest
 
+from test_bf16_parts import ROUNDING
+
 pytestmark = pytest.mark.gpu
+
+# form of a linear: (kind, columns, rows) of a workgroup
+W32, W64, W128 = (0, 32, 16), (0, 64, 16), (0, 128, 16)
+SHARED = (1, 128, 128)
+P64, P128_64, P128 = (2, 64, 64), (2, 128, 64), (2, 128, 128)
 
 
 @functools.lru_cache(maxsize=None)
-def _h1_weights(path):
+def _model(path):
     with open(path) as f:
-        return np.asarray(json.load(f)["H1_weights"])
+        d = json.load(f)
+    C = d["num_channels"]
+
+    def f32(w):
+        return np.asarray(w, np.float32).astype(np.float64)
+
+    return (C, [[f32(b).reshape(C, C) for b in w] for w in d["A0_weights"]], f32(d["H1_weights"]).reshape(-1, C, C),
+            [f32(w).reshape(-1, C) for w in d["A1_weights"]])
 
 
-def _sparse(n, seed):
+def _sparse(n, seed, choice):
     rng = np.random.default_rng(seed)
     m = int(np.ceil(n ** (1.0 / 3.0) - 1e-9))
     sites = np.stack(np.meshgrid(*(np.arange(m),) * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
-    return sites * 4.6 + rng.uniform(-0.4, 0.4, size=(n, 3)), np.eye(3) * 4.6 * m, rng.choice([8, 22, 38], size=n)
+    return sites * 4.6 + rng.uniform(-0.4, 0.4, size=(n, 3)), np.eye(3) * 4.6 * m, rng.choice(choice, size=n)
 
 
-@pytest.mark.parametrize("model,n", [("tiny", 1), ("tiny", 16), ("tiny", 43), ("tiny", 129), ("tiny", 12001),
-                                     ("medium", 1), ("medium", 15), ("medium", 17), ("medium", 128), ("medium", 1303),
-                                     ("medium", 3001), ("medium", 5003), ("medium", 17001)])
-def test_h1_linear_against_float64(model, n, tiny_model_path, medium_model_path):
+def _error(y, x, w):
+    """rms of y - x w over rms of |x| |w|"""
+    ref, scale = x @ w, np.abs(x) @ np.abs(w)
+    return np.sqrt(np.mean((y - ref) ** 2) / np.mean(scale ** 2))
+
+
+# model, atoms, forms of A0, H1, A1 and the reverse of A1
+CASES = [
+    ("tiny", 1, W32, W32, W32, W32),
+    ("tiny", 16, W32, W32, W32, W32),
+    ("tiny", 43, W32, W32, W32, W32),
+    ("tiny", 16451, W32, W32, W32, W32),
+    ("medium", 1, W64, W64, W64, W64),
+    ("medium", 15, W64, W64, W64, W64),
+    ("medium", 17, W64, W64, W64, W64),
+    ("medium", 128, W64, W64, W64, W64),
+    ("medium", 1303, W64, W64, W64, W64),
+    ("medium", 5003, W64, W64, W64, W128),
+    ("medium", 12001, W128, W64, W64, SHARED),
+    ("wide", 1, P64, P64, P64, P64),
+    ("wide", 15, P64, P64, P64, P64),
+    ("wide", 65, P64, P64, P64, P64),
+    ("wide", 129, P64, P64, P64, P64),
+    ("wide", 1203, P128_64, P64, P128_64, P128),
+    ("wide", 2501, P128, P128_64, P128, P128),
+    ("wide", 4003, P128, P128, P128, P128),
+]
+
+
+@pytest.mark.parametrize("model,n,a0,h1,a1,a1r", CASES)
+def test_linears_against_float64(request, model, n, a0, h1, a1, a1r):
     from symmetrix.mace_kokkos import MACEKokkosFloat
-    path = tiny_model_path if model == "tiny" else medium_model_path
-    pos, cell, numbers = _sparse(n, n)
+    path = request.getfixturevalue(model + "_model_path")
+    C, A0w, H1w, A1w = _model(path)
     ev = MACEKokkosFloat(path)
+    pos, cell, numbers = _sparse(n, n, [1, 8] if model == "wide" else [8, 22, 38])
     lut = {z: i for i, z in enumerate(ev.atomic_numbers)}
     types = np.array([lut[int(z)] for z in numbers], np.int32)
     g = ev._prepare_periodic_factorized_graph(types, pos, cell, np.linalg.inv(cell), ev.r_cut + 0.5)
     ev._compute_prepared_factorized_positions(g["generation"], pos)
-    C, L = ev.num_channels, ev.L_max
-    m0 = ev._stage("M0").reshape(n, (L + 1) ** 2, C).astype(np.float64)
-    h1 = ev._stage("H1").reshape(n, (L + 1) ** 2, C)
-    w = _h1_weights(path).reshape(L + 1, C, C)
-    assert np.abs(m0).max() > 0
-    for l in range(L + 1):
-        x = m0[:, l * l:(l + 1) ** 2]
-        bound = (C + 1) * 2.0 ** -24 * (np.abs(x) @ np.abs(w[l])) + 1e-30
-        assert np.all(np.abs(h1[:, l * l:(l + 1) ** 2] - x @ w[l]) <= bound)
+    forms = [tuple(int(v) for v in f) for f in ev._stage("linear_forms").reshape(4, 3)]
+    print(model, n, forms, flush=True)
+    assert forms == [a0, h1, a1, a1r]
+
+    def stage(name):
+        return ev._stage(name).reshape(n, -1, C).astype(np.float64)
+
+    phi0, A0, m0, H1 = (stage(s) for s in ("Phi0", "A0", "M0", "H1"))
+    phi1, A1, A1_adj, dphi1 = (stage(s) for s in ("Phi1", "A1", "A1_adj", "dPhi1"))
+    errors, base = {}, 0
+    for l in range(ev.l_max + 1):
+        rows = slice(l * l, (l + 1) ** 2)
+        for t in np.unique(types):
+            errors["A0", l, t] = _error(A0[types == t][:, rows], phi0[types == t][:, rows], A0w[t][l])
+        if l <= ev.L_max:
+            errors["H1", l] = _error(H1[:, rows], m0[:, rows], H1w[l])
+        K = len(A1w[l])
+        cols = slice(base, base + (2 * l + 1) * K // C)  # Phi1 rows of an l: m, then its paths
+        base = cols.stop
+        errors["A1", l] = _error(A1[:, rows], phi1[:, cols].reshape(n, 2 * l + 1, K), A1w[l])
+        errors["A1 reverse", l] = _error(dphi1[:, cols].reshape(n, 2 * l + 1, K), A1_adj[:, rows], A1w[l].T)
+    print("largest rms error %.2e (%s)" % max((e, k) for k, e in errors.items()), flush=True)
+    assert max(errors.values()) <= ROUNDING
 
 
 def test_values_beyond_bf16_and_infinities_at_256_channels(wide_model_path, tmp_path):
