@@ -1205,14 +1205,16 @@ __global__ __launch_bounds__(64 * kGemmShareWaves) void k_node_gemm_shared(
 // out as products of bf16 parts (split_operand, v_mfma_f32_16x16x32_bf16 with
 // FP32 accumulators).  Six such MFMAs cover 32 input channels in 96 cycles
 // where the FP32 form needs 256, and 24 accumulator updates instead of 32 round
-// a sum of 128 terms.
+// a sum of 128 terms.  Six linears of 30,000 nodes (256 channels, L_max 2) 4.5
+// ms, 40% MFMA busy; 6.7 ms on FP32 MFMAs at 72%.  Root mean square error of a
+// sum against 64 bits 4e-8 of its sum |x w|, 5e-8 in FP32 products.
 //
 // A workgroup of four waves takes RT consecutive 16-row tiles a wave of one
 // GemmTileSet (the set with two, its halves with one) and 16*NSUB columns.
 // The weights, split and put in operand order when the model is loaded
 // (launch_pack_gemm_weights), cross LDS once per workgroup and 32-channel
 // chunk, the next chunk's weights and rows in flight while one runs; a wave
-// splits its own rows (44 VALU instructions a tile and chunk against 12*NSUB
+// splits its own rows (60 VALU instructions a tile and chunk against 6*NSUB
 // MFMAs).  In a tile, lane l supplies channels 4*(l/16).. +3 and 16 + 4*(l/16).. +3 of
 // row or column l%16 (any order will do, the same for both; this one reads 64
 // contiguous bytes a row) and holds columns 4*(l/16).. +3 of row l%16.  Rows

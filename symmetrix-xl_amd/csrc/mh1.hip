@@ -638,7 +638,7 @@ __global__ __launch_bounds__(256) void k_mlp_reverse(const DMlp m, const DRadial
 // a LayerNorm's row sums are the lane's 16 units plus two cross-group shuffles.
 // In FP32 products (v_mfma_f32_16x16x4_f32) the MFMAs were the larger half of
 // these kernels' issue time; the parts' six MFMAs take 96 cycles for 32
-// channels where the FP32 form takes 256, and split the activations with 44
+// channels where the FP32 form takes 256, and split the activations with 60
 // VALU instructions an edge tile and chunk.  At 184,320 edges (40-64-64-64-128
 // and -320): forward 338 -> 224 us, output reverse 202 -> 158, reverse 351 ->
 // 252.  What is left is LayerNorm and SiLU, the weights' way through L1 (138 KB
