@@ -150,7 +150,7 @@ struct GemmTileSet {
     int row_start, rows, group;
 };
 // Channels from which a model's node linears run as products of bf16 parts
-// (the reason stands at launch_node_gemm).
+// (the reason stands at node_gemm_form).
 constexpr int kGemmPartsChannels = 256;
 struct GemmPlan {
     const GemmTile* tiles = nullptr;
